@@ -10,7 +10,12 @@
 // fp32 throughout; results are tolerance-class against the reference (its exp
 // is a Cephes polynomial, its sums run in another order).
 //
-// A block owns 16 queries of one head; its W waves split the key range: wave w
+// Two kernels: attn_split (below, head_dim <= 128) forms both products from
+// fp16 parts of the fp32 values, attn_fwd from the values themselves on the
+// fp32 matrix cores; it keeps head_dim 129 to 256 and the calls the split form
+// does not take (scale 0 or not finite, strides or lengths past its offsets).
+//
+// attn_fwd: a block owns 16 queries of one head; its W waves split the key range: wave w
 // takes key tiles w, w + W, ... (KT keys each), stages each tile in its own
 // LDS region (no block barrier in the main loop) and keeps its own online
 // softmax state; at the end the waves merge their (max, sum, output) through
@@ -32,9 +37,10 @@
 // the reference forms them); exp(x) is evaluated as v_exp_f32(x * log2 e).
 
 #include "common.h"
+#include "wave.h"
 
 #include <cfloat>
-#include <cstdlib>
+#include <cmath>
 
 namespace vla {
 namespace hip {
@@ -112,11 +118,11 @@ __global__ __launch_bounds__(W * 64) void attn_fwd(AttnArgs a) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, c = lane & 15;
-    // XCD-aware block order for grids of at most one round (256 blocks; ACT,
-    // SmolVLA): the hardware deals workgroup i to XCD i % 8, so each XCD is
-    // given a contiguous run of (head, query tile) pairs and its L2 holds the
-    // K/V rows of a few heads instead of every head's. Larger grids (Octo,
-    // SigLIP) measured slower that way; they take the balanced order below.
+    // XCD-aware block order for grids of at most one round (256 blocks): the
+    // hardware deals workgroup i to XCD i % 8, so each XCD is given a contiguous
+    // run of (head, query tile) pairs and its L2 holds the K/V rows of a few
+    // heads instead of every head's. Larger grids measured slower that way;
+    // they take the balanced order below.
     const int nqt = gridDim.x, total = nqt * gridDim.y;
     const int bid = blockIdx.y * nqt + blockIdx.x;
     int qt, h;
@@ -125,10 +131,9 @@ __global__ __launch_bounds__(W * 64) void attn_fwd(AttnArgs a) {
         const int logical = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
         qt = logical % nqt;
         h = logical / nqt;
-    } else if constexpr (W <= 4) {
-        // grids of 1.5+ blocks per CU take 4 waves per block (run_attn). Rounds
-        // of 256 blocks put one block on every CU (block b and b + 256 share a
-        // CU); under causal and block-causal masks a query tile's work grows
+    } else {
+        // rounds of 256 blocks put one block on every CU (block b and b + 256
+        // share a CU); under causal and block-causal masks a query tile's work grows
         // with its index, so tiles are dealt heaviest first with every other
         // round reversed: a CU's heavy block meets a light one, and a last
         // partial round gets the lightest
@@ -137,9 +142,6 @@ __global__ __launch_bounds__(W * 64) void attn_fwd(AttnArgs a) {
         const int i = total - 1 - (start + ((r & 1) ? len - 1 - p : p));
         qt = i / gridDim.y;
         h = i - qt * gridDim.y;
-    } else {
-        qt = bid % nqt;
-        h = bid / nqt;
     }
     const int kvh = h / (a.n_q / a.n_kv);
     const int HD = a.head_dim;
@@ -508,37 +510,826 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
     else launch_kd<HDP, KT, W, 0>(a, st);
 }
 
-// VLA_HIP_ATTN_W=<1|2|4|8> forces the waves per block (A/B runs; the values
-// only change by fp32 summation order across waves).
-int forced_waves() {
-    static const int w = [] {
-        const char* e = std::getenv("VLA_HIP_ATTN_W");
-        const int v = e ? std::atoi(e) : 0;
-        return v == 1 || v == 2 || v == 4 || v == 8 ? v : 0;
-    }();
-    return w;
+// ---------------------------------------------------------------------------
+// attn_split: the same attention with both products on the fp16 matrix cores.
+//
+// Scaled by a power of two, a float x is h + m + e with h = fp16(x), m =
+// fp16(x - h) and |e| <= 2^-22 |x| (2^-24.5 in the mean, and no more than 2^-40
+// of the largest value that shares the scale, fp16's subnormals included). A
+// product of two floats is hh + hm + mh to that accuracy, so three
+// v_mfma_f32_16x16x32_f16 (16 cycles each, exact products, fp32 sums over 32
+// terms at once) replace the eight v_mfma_f32_16x16x4_f32 (32 cycles each) of a
+// 16 x 16 x 32 product, and the sums round an eighth as often: against 64 bits
+// the outputs are closer than the fp32 matrix cores' (2-norm, 1024 x 1024 x 12 heads of 64,
+// N(0, 1): 2.3e-7 against 4.1e-7; 50 x 227 x 15: 2.0e-7 against 3.0e-7).
+// Scales: one per query row, one per tile for K, a running one per wave for V
+// (its accumulators are rescaled with it, as for a new maximum), 2^15 for the
+// weights; all powers of two, taken out again exactly.
+//
+// A block owns 16 * QF queries of one head and its W waves split the key
+// range in tiles of 32 keys (tile t, t + W, ...), each wave for all of the
+// block's queries, so every K and V value is loaded and split once per block.
+// Every global load puts the 16 lanes of a group on 256 contiguous bytes of a
+// key row. (Loading K in the matrix cores' operand order, 16 rows by 16 bytes
+// across neighbouring lanes, costs the address unit a cycle per lane: 14.7
+// bytes per clock and CU against 40, measured from L2.) K's parts cross the
+// lanes through a wave's own LDS rows; V's do not have to, since the k index of
+// a product may run over its terms in any order as long as both operands use
+// the same one:
+//   S^T = K Q^T   : lane (g = l / 16, c = l % 16) supplies key c, dims 8 g ..
+//                   8 g + 7 of a 32-dim step;
+//   O^T = V^T P^T : element i of lane group g is key 16 (i / 4) + 4 g + i % 4,
+//                   which is the probability the lane already holds from S^T
+//                   (sub-tile i / 4, register i % 4), and V's row index c of
+//                   16-row tile dt stands for dim 4 c + dt, so a lane's own
+//                   float4 loads of eight key rows are its operands.
+// The loads of a wave's next tile are issued as soon as the registers of this
+// one are split.
+//
+// Infinities (and NaN) in an operand: such a block is computed again from the
+// inputs in plain fp32 (attn_block_f32).
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+struct Split8 {
+    f16x8 h, m;
+};
+
+// The two parts of x0 and x1, packed. (v_fma_mix{lo,hi}_f16 would scale, round
+// and subtract at once, but they issue at half rate: 8 cycles against 4 for
+// v_cvt_pk_f16_f32 and v_fma_mix_f32.)
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m) {
+    float r0, r1;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(x0), "v"(x1));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(h), "v"(x0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(h), "v"(x1));
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(m) : "v"(r0), "v"(r1));
+}
+__device__ __forceinline__ Split8 split8(const float4& x, const float4& y) {
+    uint4 h, m;
+    split2(x.x, x.y, h.x, m.x);
+    split2(x.z, x.w, h.y, m.y);
+    split2(y.x, y.y, h.z, m.z);
+    split2(y.z, y.w, h.w, m.w);
+    return Split8{__builtin_bit_cast(f16x8, h), __builtin_bit_cast(f16x8, m)};
+}
+__device__ __forceinline__ Split8 split8(const float4& x, const float4& y, float s) {
+    return split8(make_float4(x.x * s, x.y * s, x.z * s, x.w * s), make_float4(y.x * s, y.y * s, y.z * s, y.w * s));
 }
 
-// W: enough waves that each walks a few key tiles, capped at WMAX (LDS).
-template <int HDP, int KT, int WMAX>
+// max(m, |x|, |y|); NaN is passed over
+__device__ __forceinline__ float absmax(float m, float x, float y) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x), "v"(y));
+    return m;
+}
+
+// max over eight values (NaN is passed over)
+__device__ __forceinline__ float max4(v4f x, v4f y) {
+    float m;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(x[0]), "v"(x[1]), "v"(x[2]));
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(m) : "v"(x[3]), "v"(y[0]));
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(m) : "v"(y[1]), "v"(y[2]));
+    return fmaxf(m, y[3]);
+}
+
+// Biased exponent of the power of two that brings values up to `mx` below 2^15
+// (fp16 ends at 65504); 254 minus it is its inverse's. Zero and the smallest
+// values take the largest that has an inverse.
+__device__ __forceinline__ uint32_t scale_exp(float mx) {
+    const uint32_t e = (__float_as_uint(mx) >> 23) & 0xffu;
+    return e < 15 ? 253u : 268u - e;
+}
+__device__ __forceinline__ bool not_finite(float mx) { return ((__float_as_uint(mx) >> 23) & 0xffu) == 255u; }
+__device__ __forceinline__ float exp_float(uint32_t e) { return __uint_as_float(e << 23); }
+
+// n / d for 0 <= n < 2^20, given the float nearest 1 / d: (n + 0.5) / d is at
+// least 0.5 / d away from the whole numbers, the rounding below n 2^-23 / d
+struct AttnInv {
+    float nqt, heads, group;  // 1 / query tiles, 1 / query heads, 1 / (query heads per kv head)
+};
+__device__ __forceinline__ int quotient(int n, float inv) {
+    return __builtin_amdgcn_readfirstlane((int)(((float)n + 0.5f) * inv));
+}
+
+__device__ __forceinline__ v4f mfma_f16(const f16x8& a, const f16x8& b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// whether query qi may not see key j (qi < seq_q, j < seq_k); *add is the
+// additive mask value of a key it may see
+__device__ __forceinline__ bool mask_blocks(const AttnArgs& a, int qi, int j, float* add) {
+    *add = 0.0f;
+    if (a.mask_kind == 1) {
+        const float mv = a.mask[(size_t)qi * a.ldm + j];
+        *add = mv;
+        return mv == -FLT_MAX;
+    }
+    if (a.mask_kind == 2) return j > qi + a.causal_offset;
+    if (a.mask_kind == 3) return !a.allow[(int)a.q_group[qi] * a.n_groups + a.k_group[j]];
+    return false;
+}
+
+// The block's queries [q0, q0 + nq) of head h in plain fp32, one query per wave
+// at a time, lanes over keys, then over dims: for operands the split kernel
+// does not carry, whose speed does not matter.
+template <int HDP>
+__device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq, int h, int kvh) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int HD = a.head_dim;
+    for (int q = wave; q < nq; q += nw) {
+        const int qi = q0 + q;
+        if (qi >= a.seq_q) break;
+        const float* qp = a.Q + (size_t)qi * a.ldq + h * HD;
+        auto score = [&](int j) {
+            float add;
+            if (mask_blocks(a, qi, j, &add)) return -INFINITY;
+            const float* kp = a.K + (size_t)j * a.ldk + kvh * HD;
+            float s = 0.0f;
+            for (int d = 0; d < HD; d++) s = fmaf(qp[d], kp[d], s);
+            s *= a.scale;
+            return a.mask_kind == 1 ? s + add : s;
+        };
+        float m = -INFINITY;
+        for (int j = lane; j < a.seq_k; j += 64) m = fmaxf(m, score(j));
+        for (int o = 32; o; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        const bool masked = m == -INFINITY;
+        float l = 0.0f;
+        float o[HDP / 64];
+#pragma unroll
+        for (int u = 0; u < HDP / 64; u++) o[u] = 0.0f;
+        for (int j0 = 0; j0 < a.seq_k; j0 += 64) {
+            const int j = j0 + lane;
+            float p = 0.0f;
+            if (j < a.seq_k) p = masked ? 1.0f : fast_exp2((score(j) - m) * kLog2e);
+            l += p;
+            const int n = a.seq_k - j0 < 64 ? a.seq_k - j0 : 64;
+            for (int t = 0; t < n; t++) {
+                const float pt = __shfl(p, t);
+#pragma unroll
+                for (int u = 0; u < HDP / 64; u++) {
+                    const int d = u * 64 + lane;
+                    if (d < HD) o[u] = fmaf(pt, a.V[(size_t)(j0 + t) * a.ldv + kvh * HD + d], o[u]);
+                }
+            }
+        }
+        for (int x = 32; x; x >>= 1) l += __shfl_xor(l, x);
+#pragma unroll
+        for (int u = 0; u < HDP / 64; u++) {
+            const int d = u * 64 + lane;
+            if (d < HD) a.out[(size_t)qi * a.ldo + h * HD + d] = o[u] / l;
+        }
+    }
+}
+
+template <int HDP, int QF, int W>
+struct SplitCfg {
+    static constexpr int S = HDP / 32;             // 32-dim steps of Q K^T
+    static constexpr int U = HDP / 64;             // 64-dim column groups of V
+    static constexpr int MO = HDP + 4;             // merge row, floats
+    static constexpr bool QLDS = QF > 2;           // the query fragments live in LDS
+    static constexpr int QB = QLDS ? QF * S * 2 * 1024 : 0;
+    static constexpr int KG = 4096;                // key groups kept in LDS behind them
+    static constexpr int FSB = QB + KG + 32;       // (a last tile reads groups past seq_k)
+    static constexpr int KROW = 2 * HDP + 16;      // bytes of one part of a key row: 16 rows'
+                                                   // 16-byte reads fall on distinct banks
+    static constexpr int KB = FSB + (QLDS ? 64 * QF : 0);  // 32 keys' two parts per wave
+    static constexpr int MAINB = KB + W * 32 * 2 * KROW;
+    static constexpr int MERGE = 4 * W * 16 * QF * (MO + 2);
+    static constexpr int MEAN = 4 * (W * 4 + 1) * HDP;  // partial means of V, then the mean
+    static constexpr int MAX0 = MERGE > MAINB ? MERGE : MAINB;
+    static constexpr int LDS = (MAX0 > MEAN ? MAX0 : MEAN) + 16;
+    static_assert(LDS <= 160 * 1024, "LDS");
+};
+
+template <int HDP, int QF, int W, int MKC, bool FULL>
+__global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs a, AttnInv inv) {
+    using C = SplitCfg<HDP, QF, W>;
+    constexpr int S = C::S, U = C::U, MO = C::MO, NQ = 16 * QF;
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    uint32_t* flags = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(smem) + C::LDS - 16);
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar addresses
+    const int g = lane >> 4, c = lane & 15;
+    // block order: as attn_fwd (XCD-contiguous up to one round of 256 blocks,
+    // else heaviest query tiles first with every other round reversed). The
+    // quotients are taken with the launch's reciprocals: exact for the block
+    // counts the launch allows, and four integer divisions ahead of the first
+    // load are not.
+    const int nqt = gridDim.x, total = nqt * gridDim.y;
+    const int bid = blockIdx.y * nqt + blockIdx.x;
+    int qt, h;
+    if (total <= 256) {
+        const int xcd = bid & 7, per = total >> 3, rem = total & 7;
+        const int logical = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
+        h = quotient(logical, inv.nqt);
+        qt = logical - h * nqt;
+    } else {
+        const int r = bid >> 8, p = bid & 255, start = r << 8;
+        const int len = total - start < 256 ? total - start : 256;
+        const int i = total - 1 - (start + ((r & 1) ? len - 1 - p : p));
+        qt = quotient(i, inv.heads);
+        h = i - qt * gridDim.y;
+    }
+    const int kvh = quotient(h, inv.group);
+    const int HD = a.head_dim;
+    const int q0 = qt * NQ;
+    const bool qfull = q0 + NQ <= a.seq_q;
+    const float* Kb = a.K + kvh * HD;
+    const float* Vb = a.V + kvh * HD;
+    if (tid == 0) *flags = 0;
+
+    // this lane's share of a tile: K rows 4 jj + g, V rows of keys
+    // 16 (jj / 4) + 4 g + jj % 4, dims 64 u + 4 c .. (rows past the last key
+    // repeat it, their scores are blocked; dims past the head read as zero)
+    float4 kr[8][U], vr[8][U];
+    const int jmax = a.seq_k - 1;
+    // base + a 32-bit byte offset per lane: rows are clamped as offsets, so a
+    // tile's last rows take no branch and no 64-bit address per lane
+    auto rload = [&](float4 (&dst)[U], const float* base, uint32_t off) {
+        const char* p = reinterpret_cast<const char*>(base);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (FULL) {
+                dst[u] = *reinterpret_cast<const float4*>(p + off + 256 * u);
+            } else {
+                const int d = 64 * u + 4 * c;
+                dst[u] = *reinterpret_cast<const float4*>(p + (off - 16u * c + 4u * min(d, HD - 4)));
+                if (d >= HD) dst[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        }
+    };
+    const uint32_t kld = 4u * a.ldk, vld = 4u * a.ldv;
+    const uint32_t koff = g * kld + 16u * c, voff = 4 * g * vld + 16u * c;
+    auto kload = [&](int kv0) {
+        const uint32_t last = min(jmax - kv0, 31) * kld + 16u * c;
+        uint32_t o = koff;
+        asm volatile("" : "+v"(o));  // eight sums here, not eight registers kept over the loop
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++) rload(kr[jj], Kb + (size_t)kv0 * a.ldk, min(o + 4 * jj * kld, last));
+    };
+    auto vload = [&](int kv0) {
+        const uint32_t last = min(jmax - kv0, 31) * vld + 16u * c;
+        uint32_t o = voff;
+        asm volatile("" : "+v"(o));
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++)
+            rload(vr[jj], Vb + (size_t)kv0 * a.ldv, min(o + (16 * (jj >> 2) + (jj & 3)) * vld, last));
+    };
+    char* kw = reinterpret_cast<char*>(smem) + C::KB + wave * (32 * 2 * C::KROW);
+
+    // keys past kv_end are blocked for every query of the block (causal bound)
+    int kv_end = a.seq_k;
+    const int mk = a.mask_kind;
+    if (mk == 2) {
+        const int qlast = (q0 + NQ < a.seq_q ? q0 + NQ : a.seq_q) - 1;
+        const int e = qlast + a.causal_offset + 1;
+        kv_end = e < 0 ? 0 : (e < kv_end ? e : kv_end);
+    }
+    const int nkt = (kv_end + 31) / 32;
+
+    // the query fragments: query 16 f + c, dims 32 s + 8 g ..
+    Split8 qreg[C::QLDS ? 1 : QF][C::QLDS ? 1 : S];
+    float fs[QF];  // scores' unit of a query, times the softmax scale and log2 e
+    f16x8* qlds = reinterpret_cast<f16x8*>(smem);
+    float* fsl = reinterpret_cast<float*>(reinterpret_cast<char*>(smem) + C::FSB);
+    auto qload = [&](int f, float4 (&x)[S][2]) {
+        const int qi = min(q0 + 16 * f + c, a.seq_q - 1);
+        const float* p = a.Q + (size_t)qi * a.ldq + h * HD;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int d = 32 * s + 8 * g + 4 * e;
+                x[s][e] = *reinterpret_cast<const float4*>(p + (FULL ? d : min(d, HD - 4)));
+                if (!FULL && d >= HD) x[s][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+    };
+    bool bad = false;
+    // splits a query fragment; returns its scores' unit times the softmax scale
+    // and log2 e
+    auto qsplit = [&](const float4 (&x)[S][2], Split8 (&q)[S]) {
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) mx = absmax(absmax(mx, x[s][e].x, x[s][e].y), x[s][e].z, x[s][e].w);
+        mx = rows_max(mx);
+        bad = bad || not_finite(mx);
+        const uint32_t e = scale_exp(mx);
+#pragma unroll
+        for (int s = 0; s < S; s++) q[s] = split8(x[s][0], x[s][1], a.scale < 0.0f ? -exp_float(e) : exp_float(e));
+        return exp_float(254u - e) * fabsf(a.scale) * kLog2e;
+    };
+    // the queries' loads ahead of the first tile's: loads return in order
+    const bool qmine = !C::QLDS || wave < QF;
+    float4 qx[C::QLDS ? 1 : QF][S][2];
+    static_assert(!C::QLDS || W >= QF, "a wave per query fragment");
+    if (qmine) {
+#pragma unroll
+        for (int f = 0; f < (C::QLDS ? 1 : QF); f++) qload(C::QLDS ? wave : f, qx[f]);
+    }
+    if (MKC != 3 && wave < nkt) {  // group masks first find a tile with something to see
+        kload(wave * 32);
+        vload(wave * 32);
+    }
+    if constexpr (C::QLDS) {
+        if (qmine) {
+            Split8 q[S];
+            const float u = qsplit(qx[0], q);
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                qlds[((wave * S + s) * 2 + 0) * 64 + lane] = q[s].h;
+                qlds[((wave * S + s) * 2 + 1) * 64 + lane] = q[s].m;
+            }
+            if (g == 0) fsl[16 * wave + c] = u;
+        }
+    } else {
+#pragma unroll
+        for (int f = 0; f < QF; f++) fs[f] = qsplit(qx[f], qreg[f]);
+    }
+
+    // group masks: the key groups a query's group may see, as two words for up
+    // to 64 groups (more are read from the table per score), and the keys'
+    // groups in LDS where they fit
+    const int G = a.n_groups;
+    uint32_t am0[QF], am1[QF];
+    int qg[QF];
+    uint8_t* kgl = reinterpret_cast<uint8_t*>(smem) + C::QB;
+    if constexpr (MKC == 3) {
+        for (int j = tid; j < a.seq_k && a.seq_k <= C::KG; j += W * 64) kgl[j] = a.k_group[j];
+#pragma unroll
+        for (int f = 0; f < QF; f++) {
+            const int qi = q0 + 16 * f + c;
+            qg[f] = qi < a.seq_q ? a.q_group[qi] : 0;
+            uint32_t lo = 0, hi = 0;
+            if (G <= 64 && qi < a.seq_q)
+                for (int x = g; x < G; x += 4) {  // the four lanes of a query read a quarter of its row each
+                    const uint32_t b = a.allow[qg[f] * G + x] ? 1u : 0u;
+                    if (x < 32) lo |= b << x;
+                    else hi |= b << (x - 32);
+                }
+            lo |= __shfl_xor(lo, 16);
+            hi |= __shfl_xor(hi, 16);
+            am0[f] = lo | __shfl_xor(lo, 32);
+            am1[f] = hi | __shfl_xor(hi, 32);
+        }
+    }
+    const bool vec_mask = MKC == 1 && (reinterpret_cast<uintptr_t>(a.mask) & 15) == 0 && (a.ldm & 3) == 0;
+    __syncthreads();
+    if constexpr (C::QLDS)
+#pragma unroll
+        for (int f = 0; f < QF; f++) fs[f] = fsl[16 * f + c];
+
+    float M[QF], lsum[QF];  // running max (times log2 e) and sum per query 16 f + c
+    v4f oacc[QF][U][4];     // O^T: dim 64 u + 4 (4 g + r) + dt of query 16 f + c,
+                            // in units of 1 / sv (both sums carry the weights' 2^15)
+    // K's and V's scales: the first tile's, until a value outgrows them (V's
+    // accumulators are then rescaled; a tile of smaller values keeps the unit)
+    float sk = 0.0f, uk = 0.0f, sv = 0.0f, uv = 0.0f, klim = -1.0f, vlim = -1.0f;
+#pragma unroll
+    for (int f = 0; f < QF; f++) {
+        M[f] = -INFINITY;
+        lsum[f] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) oacc[f][u][dt] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // group masks: bit 8 f + 4 kt + r says whether this lane's score of tile t
+    // is blocked. A tile the table blocks for every query would add p = 0
+    // everywhere: it is neither loaded nor computed.
+    constexpr uint32_t kAll = QF == 4 ? 0xffffffffu : (1u << (8 * QF)) - 1u;
+    auto dead_of = [&](int kv0) {
+        uint32_t dead = 0;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+            const int j0 = kv0 + 16 * kt + 4 * g;
+            uint32_t kg = 0;
+            if (a.seq_k <= C::KG) kg = *reinterpret_cast<const uint32_t*>(kgl + j0);
+            else
+                for (int r = 0; r < 4; r++) kg |= (uint32_t)a.k_group[min(j0 + r, jmax)] << (8 * r);
+            if (G <= 64) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t v = (kg >> (8 * r)) & 0xffu;
+#pragma unroll
+                    for (int f = 0; f < QF; f++) {
+                        const uint32_t w = v < 32 ? am0[f] : am1[f];
+                        dead |= (~(w >> (v & 31)) & 1u) << (8 * f + 4 * kt + r);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int f = 0; f < QF; f++)
+                    for (int r = 0; r < 4; r++)
+                        if (!a.allow[qg[f] * G + (int)((kg >> (8 * r)) & 0xffu)]) dead |= 1u << (8 * f + 4 * kt + r);
+            }
+            // keys past the last one
+            const int past = j0 + 4 - a.seq_k;
+            const uint32_t out = past <= 0 ? 0u : (0xf0u >> (past > 4 ? 4 : past)) & 0xfu;
+#pragma unroll
+            for (int f = 0; f < QF; f++) dead |= out << (8 * f + 4 * kt);
+        }
+#pragma unroll
+        for (int f = 0; f < QF; f++)
+            if (q0 + 16 * f + c >= a.seq_q) dead |= 0xffu << (8 * f);
+        return dead;
+    };
+    // the first tile from t on (in steps of W) with something to see
+    auto next_tile = [&](int t, uint32_t* dead) {
+        if constexpr (MKC == 3) {
+            for (; t < nkt; t += W) {
+                *dead = dead_of(t * 32);
+                if (__any(*dead != kAll)) break;
+            }
+        }
+        return t;
+    };
+
+    uint32_t dead = 0;
+    int t = next_tile(wave, &dead);
+    if (MKC == 3 && t < nkt) {
+        kload(t * 32);
+        vload(t * 32);
+    }
+    while (t < nkt) {
+        const int kv0 = t * 32;
+        uint32_t dead_next = 0;
+        const int tn = next_tile(t + W, &dead_next);
+        const bool more = tn < nkt;
+        float mval[MKC == 1 ? QF : 1][2][4];
+        if constexpr (MKC == 1) {
+#pragma unroll
+            for (int f = 0; f < QF; f++)
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++) {
+                    const int qi = q0 + 16 * f + c, j0 = kv0 + 16 * kt + 4 * g;
+                    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (qi < a.seq_q) {
+                        const float* mp = a.mask + (size_t)qi * a.ldm + j0;
+                        if (j0 + 4 <= a.seq_k && vec_mask) {
+                            v = *reinterpret_cast<const float4*>(mp);
+                        } else {
+                            if (j0 < a.seq_k) v.x = mp[0];
+                            if (j0 + 1 < a.seq_k) v.y = mp[1];
+                            if (j0 + 2 < a.seq_k) v.z = mp[2];
+                            if (j0 + 3 < a.seq_k) v.w = mp[3];
+                        }
+                    }
+                    mval[f][kt][0] = v.x;
+                    mval[f][kt][1] = v.y;
+                    mval[f][kt][2] = v.z;
+                    mval[f][kt][3] = v.w;
+                }
+        }
+
+        float kmax = 0.0f;
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                kmax = absmax(absmax(kmax, kr[jj][u].x, kr[jj][u].y), kr[jj][u].z, kr[jj][u].w);
+        if (__any(kmax > klim)) {
+            kmax = wave_max_f32(kmax);
+            bad = bad || not_finite(kmax);
+            const uint32_t e = scale_exp(kmax);
+            sk = exp_float(e);
+            uk = exp_float(254u - e);
+            klim = 32768.0f * uk;
+        }
+
+        // K's parts to the operand's lanes through this wave's LDS rows
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++)
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                uint2 kh, km;
+                split2(kr[jj][u].x * sk, kr[jj][u].y * sk, kh.x, km.x);
+                split2(kr[jj][u].z * sk, kr[jj][u].w * sk, kh.y, km.y);
+                char* p = kw + (4 * jj + g) * (2 * C::KROW) + 128 * u + 8 * c;
+                *reinterpret_cast<uint2*>(p) = kh;
+                *reinterpret_cast<uint2*>(p + C::KROW) = km;
+            }
+        if (more) kload(tn * 32);
+        wave_lds_sync();
+
+        // S^T = K Q^T
+        v4f sacc[QF][2];
+#pragma unroll
+        for (int f = 0; f < QF; f++) sacc[f][0] = sacc[f][1] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            Split8 kp[2], q[QF];
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++) {
+                const char* p = kw + (16 * kt + c) * (2 * C::KROW) + 64 * s + 16 * g;
+                kp[kt].h = *reinterpret_cast<const f16x8*>(p);
+                kp[kt].m = *reinterpret_cast<const f16x8*>(p + C::KROW);
+            }
+#pragma unroll
+            for (int f = 0; f < QF; f++) {
+                if constexpr (C::QLDS) {
+                    q[f].h = qlds[((f * S + s) * 2 + 0) * 64 + lane];
+                    q[f].m = qlds[((f * S + s) * 2 + 1) * 64 + lane];
+                } else {
+                    q[f] = qreg[f][s];
+                }
+            }
+#define VLA_QK(KP, QP)                                       \
+    _Pragma("unroll") for (int f = 0; f < QF; f++)           \
+        _Pragma("unroll") for (int kt = 0; kt < 2; kt++)     \
+            sacc[f][kt] = mfma_f16(kp[kt].KP, q[f].QP, sacc[f][kt]);
+            VLA_QK(m, h)
+            VLA_QK(h, m)
+            VLA_QK(h, h)
+#undef VLA_QK
+        }
+        float vmax = 0.0f, resc = 1.0f;
+#pragma unroll
+        for (int jj = 0; jj < 8; jj++)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                vmax = absmax(absmax(vmax, vr[jj][u].x, vr[jj][u].y), vr[jj][u].z, vr[jj][u].w);
+        if (__any(vmax > vlim)) {
+            vmax = wave_max_f32(vmax);
+            bad = bad || not_finite(vmax);
+            const uint32_t e = scale_exp(vmax);
+            sv = exp_float(e);
+            resc = uv * sv;  // the old unit over the new one (0 before any tile, whose sums are 0)
+            uv = exp_float(254u - e);
+            vlim = 32768.0f * uv;
+        }
+
+        // scale, mask and online softmax in the log2 domain: t = acc f + mask
+        // log2 e, p = 2^(t - M) with one rounding in the exponent; the rounding
+        // of M is common to a query's weights and leaves with the division
+        Split8 pp[QF];
+        const bool plain = MKC == 0 && mk == 0 && qfull && kv0 + 32 <= kv_end;  // wave-uniform
+#pragma unroll
+        for (int f = 0; f < QF; f++) {
+            const int qi = q0 + 16 * f + c;
+            const float fq = fs[f] * uk;  // > 0
+            float mt;
+            if constexpr (MKC == 1) {
+                mt = -INFINITY;
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float v = mval[f][kt][r];
+                        const bool blocked =
+                            qi >= a.seq_q || kv0 + 16 * kt + 4 * g + r >= kv_end || v == -FLT_MAX;
+                        mval[f][kt][r] = blocked ? -INFINITY : v * kLog2e;
+                        mt = fmaxf(mt, fmaf(sacc[f][kt][r], fq, mval[f][kt][r]));
+                    }
+            } else {
+                if (!plain) {
+#pragma unroll
+                    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const int j = kv0 + 16 * kt + 4 * g + r;
+                            const bool blocked =
+                                MKC == 3 ? (dead >> (8 * f + 4 * kt + r)) & 1u
+                                         : qi >= a.seq_q || j >= kv_end || (mk == 2 && j > qi + a.causal_offset);
+                            sacc[f][kt][r] = blocked ? -INFINITY : sacc[f][kt][r];
+                        }
+                }
+                mt = max4(sacc[f][0], sacc[f][1]) * fq;
+            }
+            const float mnew = fmaxf(M[f], rows_max(mt));
+            // a query that has seen nothing yet keeps M = -inf; its weights are
+            // 2^-inf = 0 against any finite reference
+            const float mref = fmaxf(mnew, -FLT_MAX);
+            const float decay = fast_exp2(M[f] - mref), alpha = decay * resc;
+            float4 x[2];
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++) {
+                auto weight = [&](int r) {
+                    // times 2^15 after the exponential: 15 in the exponent would coarsen it
+                    return fast_exp2(fmaf(sacc[f][kt][r], fq, MKC == 1 ? mval[f][kt][r] - mref : -mref)) * 32768.0f;
+                };
+                x[kt] = make_float4(weight(0), weight(1), weight(2), weight(3));
+            }
+            const float ps = ((x[0].x + x[0].y) + (x[0].z + x[0].w)) + ((x[1].x + x[1].y) + (x[1].z + x[1].w));
+            lsum[f] = fmaf(lsum[f], decay, ps);
+            M[f] = mnew;
+            if (__any(alpha != 1.0f)) {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int dt = 0; dt < 4; dt++) oacc[f][u][dt] *= alpha;
+            }
+            pp[f] = split8(x[0], x[1]);
+        }
+
+        // O^T += V^T P^T
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            Split8 vp[4];
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) {
+                float4 e[2];
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++) {
+                    auto at = [&](int r) {
+                        const float4& v = vr[4 * kt + r][u];
+                        return dt == 0 ? v.x : dt == 1 ? v.y : dt == 2 ? v.z : v.w;
+                    };
+                    e[kt] = make_float4(at(0), at(1), at(2), at(3));
+                }
+                vp[dt] = split8(e[0], e[1], sv);
+            }
+            if (u == U - 1 && more) vload(tn * 32);
+#define VLA_PV(VP, PP)                                       \
+    _Pragma("unroll") for (int f = 0; f < QF; f++)           \
+        _Pragma("unroll") for (int dt = 0; dt < 4; dt++)     \
+            oacc[f][u][dt] = mfma_f16(vp[dt].VP, pp[f].PP, oacc[f][u][dt]);
+            VLA_PV(m, h)
+            VLA_PV(h, m)
+            VLA_PV(h, h)
+#undef VLA_PV
+        }
+        wave_lds_sync();  // this tile's reads of kw are done before the next tile's writes
+        t = tn;
+        dead = dead_next;
+    }
+
+    if (__any(bad) && lane == 0) atomicOr(flags, 1u);
+#pragma unroll
+    for (int f = 0; f < QF; f++) lsum[f] = rows_sum(lsum[f]);
+
+    // merge the waves' partial states: M*, then sum_w 2^(M_w - M*) (l_w, O_w)
+    __syncthreads();
+    float* Mm = smem;                   // [W][NQ]
+    float* Ml = smem + W * NQ;          // [W][NQ]
+    float* Mo = smem + 2 * W * NQ;      // [W][NQ][MO]
+#pragma unroll
+    for (int f = 0; f < QF; f++) {
+        if (g == 0) {
+            Mm[wave * NQ + 16 * f + c] = M[f];
+            Ml[wave * NQ + 16 * f + c] = lsum[f];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                *reinterpret_cast<float4*>(Mo + (wave * NQ + 16 * f + c) * MO + 64 * u + 16 * g + 4 * r) =
+                    make_float4(oacc[f][u][0][r] * uv, oacc[f][u][1][r] * uv, oacc[f][u][2][r] * uv,
+                                oacc[f][u][3][r] * uv);
+    }
+    __syncthreads();
+    if (*flags) {  // block-uniform
+        attn_block_f32<HDP>(a, q0, NQ, h, kvh);
+        return;
+    }
+    // thread x writes float4 column x % (HDP / 4) of queries x / (HDP / 4), ...:
+    // whole 16-byte runs of an output row per wave
+    constexpr int QPT = W * 64 / (HDP / 4);  // queries per step of the block
+    const int d4 = tid % (HDP / 4);
+    bool any_masked = false;
+    for (int q = tid / (HDP / 4); q < NQ; q += QPT) {
+        if (q0 + q >= a.seq_q) break;
+        float mw[W], ms = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            mw[w] = Mm[w * NQ + q];
+            ms = fmaxf(ms, mw[w]);
+        }
+        if (ms == -INFINITY) {
+            any_masked = true;
+            continue;
+        }
+        float l = 0.0f;
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const float fw = mw[w] == -INFINITY ? 0.0f : fast_exp2(mw[w] - ms);
+            l += fw * Ml[w * NQ + q];
+            const float4 v = *reinterpret_cast<const float4*>(Mo + (w * NQ + q) * MO + 4 * d4);
+            o.x += fw * v.x;
+            o.y += fw * v.y;
+            o.z += fw * v.z;
+            o.w += fw * v.w;
+        }
+        const float inv = 1.0f / l;
+        if (4 * d4 < HD)
+            *reinterpret_cast<float4*>(a.out + (size_t)(q0 + q) * a.ldo + h * HD + 4 * d4) =
+                make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+    }
+    // rows with every key blocked: the uniform mean of V over all seq_k keys,
+    // the same for each of them, from partial sums over 4 W strided key sets
+    if (__syncthreads_or(any_masked)) {
+        // the partial sums take Mm's place: each thread first notes which of its
+        // queries are masked
+        uint32_t mine = 0;
+        int n = 0;
+        for (int q = tid / (HDP / 4); q < NQ; q += QPT, n++) {
+            if (q0 + q >= a.seq_q) break;
+            float ms = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < W; w++) ms = fmaxf(ms, Mm[w * NQ + q]);
+            if (ms == -INFINITY) mine |= 1u << n;
+        }
+        __syncthreads();
+        constexpr int NP = W * 64 / (HDP / 4);
+        const int part = tid / (HDP / 4);
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (4 * d4 < HD)
+            for (int j = part; j < a.seq_k; j += NP) {
+                const float4 v = *reinterpret_cast<const float4*>(Vb + (size_t)j * a.ldv + 4 * d4);
+                sum.x += v.x;
+                sum.y += v.y;
+                sum.z += v.z;
+                sum.w += v.w;
+            }
+        *reinterpret_cast<float4*>(smem + part * HDP + 4 * d4) = sum;
+        __syncthreads();
+        float4 mean = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int x = 0; x < NP; x++) {
+            const float4 v = *reinterpret_cast<const float4*>(smem + x * HDP + 4 * d4);
+            mean.x += v.x;
+            mean.y += v.y;
+            mean.z += v.z;
+            mean.w += v.w;
+        }
+        const float inv = 1.0f / (float)a.seq_k;
+        n = 0;
+        for (int q = part; q < NQ; q += QPT, n++)
+            if (((mine >> n) & 1u) && 4 * d4 < HD)
+                *reinterpret_cast<float4*>(a.out + (size_t)(q0 + q) * a.ldo + h * HD + 4 * d4) =
+                    make_float4(mean.x * inv, mean.y * inv, mean.z * inv, mean.w * inv);
+    }
+}
+
+template <int HDP, int QF, int W, int MKC, bool FULL>
+void launch_split_kd(const AttnArgs& a, hipStream_t st) {
+    using C = SplitCfg<HDP, QF, W>;
+    static const bool attr = [] {
+        if (C::LDS > 65536)
+            VLA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_split<HDP, QF, W, MKC, FULL>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
+        return true;
+    }();
+    (void)attr;
+    attn_split<HDP, QF, W, MKC, FULL>
+        <<<dim3((a.seq_q + 16 * QF - 1) / (16 * QF), a.n_q), W * 64, C::LDS, st>>>(a, {1.0f / (float)((a.seq_q + 16 * QF - 1) / (16 * QF)), 1.0f / (float)a.n_q,
+                                      1.0f / (float)(a.n_q / a.n_kv)});
+}
+
+template <int HDP, int QF, int W, bool FULL>
+void launch_split_w(const AttnArgs& a, hipStream_t st) {
+    if (a.mask_kind == 1) launch_split_kd<HDP, QF, W, 1, FULL>(a, st);
+    else if (a.mask_kind == 3) launch_split_kd<HDP, QF, W, 3, FULL>(a, st);
+    else launch_split_kd<HDP, QF, W, 0, FULL>(a, st);
+}
+
+// Query fragments and waves per block, from the sizes alone (a dense mask of
+// zeros must take the same waves as no mask: the merge order is theirs).
+// QF: the fewest 16-query fragments whose blocks fit one round of the 256 CUs
+// (a block of 8 waves, or of 4 at head_dim 128, fills a CU's registers), else
+// the most: every fragment more divides the K/V traffic and the splitting, a
+// second round costs as much as the first. Measured, us (fp32 matrix cores |
+// QF 1, 2, 3, 4): 1024 x 1024 x 12 heads 43.7 | 34.3 31.5 36.1 25.6; 690 x 690
+// x 12, block-causal 28.8 | 26.2 22.3 20.1 28.0; 512 x 512 x 12 17.6 | 14.1
+// 12.8 13.5 15.3; 302 x 302 x 8 8.3 | 8.1 10.3 10.0 12.7.
+// W: 8 waves from 9 tiles of 32 keys on, 4 for 3 to 8 (50 x 227 x 15 heads 8.9
+// against 9.2), 2 below; head_dim 128 has the registers for 4.
+template <int HDP, bool FULL>
+void run_split(const AttnArgs& a, hipStream_t st) {
+    const int tiles = (a.seq_k + 31) / 32;
+    const long frags = (a.seq_q + 15) / 16;
+    auto fits = [&](int qf) { return (frags + qf - 1) / qf * a.n_q <= 256; };
+    if constexpr (HDP == 128) {
+        if (fits(1)) launch_split_w<HDP, 1, 4, FULL>(a, st);
+        else launch_split_w<HDP, 2, 4, FULL>(a, st);
+    } else if (tiles <= 2) {
+        launch_split_w<HDP, 1, 2, FULL>(a, st);
+    } else if (tiles <= 8) {
+        if (fits(1)) launch_split_w<HDP, 1, 4, FULL>(a, st);
+        else launch_split_w<HDP, 2, 4, FULL>(a, st);
+    } else {
+        if (fits(1)) launch_split_w<HDP, 1, 8, FULL>(a, st);
+        else if (fits(2)) launch_split_w<HDP, 2, 8, FULL>(a, st);
+        else if (FULL && fits(3)) launch_split_w<HDP, FULL ? 3 : 4, 8, FULL>(a, st);
+        else launch_split_w<HDP, 4, 8, FULL>(a, st);
+    }
+    VLA_LAUNCH_CHECK();
+}
+
+// attn_fwd's waves: enough that each walks a few key tiles, at most 4 (LDS).
 void run_attn(const AttnArgs& a, hipStream_t st) {
     int kv = a.seq_k;
     if (a.mask_kind == 2) {  // keys no query of the problem can see are never walked
         const int e = a.seq_q + a.causal_offset;
         kv = e < 1 ? 1 : (e < kv ? e : kv);
     }
-    int tiles = (kv + KT - 1) / KT;
-    // grids of 1.5+ blocks per CU (Octo's 658-690 tokens x 12 heads): 4 waves,
-    // so two blocks share a CU and hide each other's load latency (measured
-    // 1.268 -> 1.235 ms and 1.457 -> 1.335 ms per Octo forward); smaller grids
-    // (ACT, SmolVLA) keep 8 waves per block (their latency grew with 4)
-    const long blocks = (long)((a.seq_q + 15) / 16) * a.n_q;
-    if (blocks >= 384 && tiles > 4) tiles = 4;
-    if (const int fw = forced_waves()) tiles = fw;
-    if (tiles <= 1) launch_w<HDP, KT, 1>(a, st);
-    else if (tiles <= 2 || WMAX == 2) launch_w<HDP, KT, 2>(a, st);
-    else if (tiles <= 4 || WMAX == 4) launch_w<HDP, KT, (WMAX < 4 ? WMAX : 4)>(a, st);
-    else launch_w<HDP, KT, WMAX>(a, st);
+    const int tiles = (kv + 15) / 16;
+    if (tiles <= 1) launch_w<256, 16, 1>(a, st);
+    else if (tiles <= 2) launch_w<256, 16, 2>(a, st);
+    else launch_w<256, 16, 4>(a, st);
     VLA_LAUNCH_CHECK();
 }
 
@@ -563,12 +1354,15 @@ void launch_attention(const AttnArgs& a, hipStream_t st) {
                                      a.n_groups <= 256),
                 "attention: group mask needs q_group, k_group, allow and 1..256 groups");
     if (a.seq_q == 0) return;
-    if (a.head_dim <= 64)
-        run_attn<64, 16, 8>(a, st);
-    else if (a.head_dim <= 128)
-        run_attn<128, 32, 4>(a, st);
-    else
-        run_attn<256, 16, 4>(a, st);
+    // scale 0 (and non-finite scales) would turn a blocked score's -inf into
+    // NaN; lengths and strides past the block index's and offsets' range
+    const bool split = std::isfinite(a.scale) && a.scale != 0.0f && a.head_dim <= 128 && a.ldk < (1 << 24) &&
+                       a.ldv < (1 << 24) && (long)((a.seq_q + 15) / 16) * a.n_q < (1 << 20);
+    if (!split) run_attn(a, st);
+    else if (a.head_dim == 64) run_split<64, true>(a, st);
+    else if (a.head_dim < 64) run_split<64, false>(a, st);
+    else if (a.head_dim == 128) run_split<128, true>(a, st);
+    else run_split<128, false>(a, st);
 }
 
 }  // namespace hip
