@@ -10,15 +10,15 @@
 // SmolVLA's flow-matching projections (src/models/smolvla/action_expert.cpp:196-211).
 // fp32 results differ from the reference's only by summation order.
 //
-// v_mfma_f32_16x16x4f32: lane l supplies A[row l % 16][k l / 16] and
-// B[col l % 16][k l / 16]; output lane l holds column l % 16, rows
-// 4 * (l / 16) + r. A block owns a BM x BN tile with four waves in a 2 x 2 grid;
-// K advances in 16-wide slabs staged through LDS (rows padded by one float so
-// the column reads of the fragment loads do not collide on a bank). M <= 128
-// takes a split-K kernel instead (see linear_f32_skinny).
+// More than 128 rows take linear_f32_tiled (two fp16 parts of every operand on
+// the fp16 matrix cores); up to 128 rows, and few tiles over a long K without a
+// workspace, linear_f32_skinny on v_mfma_f32_16x16x4f32: lane l supplies A[row
+// l % 16][k l / 16] and B[col l % 16][k l / 16]; output lane l holds column
+// l % 16, rows 4 * (l / 16) + r.
 
 #include "act.h"
 #include "common.h"
+#include "wave.h"
 
 #include <cstdlib>
 
@@ -30,107 +30,107 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void linear_f32_kernel(float* __restrict__ out, int ldo,
-                                                         const float* __restrict__ x, int ldx,
-                                                         const float* __restrict__ W, int ldw,
-                                                         const float* __restrict__ bias, int M,
-                                                         int N, int K, int act, int accumulate,
-                                                         float alpha) {
-    constexpr int BK = 16, SP = BK + 1;
-    constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
-    __shared__ float sa[BM * SP], sb[BN * SP];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+// The two fp16 parts of a float scaled by a power of two: x s = h + m + e, h =
+// fp16(x s), m = fp16(x s - h), |e| <= 2^-22 |x s| or 2^-25 (half of fp16's
+// smallest step), whichever is more.
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-    v4f acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m) {
+    float r0, r1;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(x0), "v"(x1));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(h), "v"(x0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(h), "v"(x1));
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(m) : "v"(r0), "v"(r1));
+}
 
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        for (int e = tid; e < BM * BK; e += 256) {
-            const int r = e / BK, c = e % BK, m = m0 + r, k = k0 + c;
-            sa[r * SP + c] = (m < M && k < K) ? x[(size_t)m * ldx + k] : 0.0f;
-        }
-        for (int e = tid; e < BN * BK; e += 256) {
-            const int r = e / BK, c = e % BK, n = n0 + r, k = k0 + c;
-            sb[r * SP + c] = (n < N && k < K) ? W[(size_t)n * ldw + k] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < BK; ks += 4) {
-            float af[FM], bf[FN];
-#pragma unroll
-            for (int i = 0; i < FM; i++) af[i] = sa[(wm * TM + i * 16 + (lane & 15)) * SP + ks + (lane >> 4)];
-#pragma unroll
-            for (int j = 0; j < FN; j++) bf[j] = sb[(wn * TN + j * 16 + (lane & 15)) * SP + ks + (lane >> 4)];
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
+// max(m, |x|, |y|, |z|, |w|); NaN is passed over
+__device__ __forceinline__ float absmax4(float m, const float4& v) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.x), "v"(v.y));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.z), "v"(v.w));
+    return m;
+}
 
-#pragma unroll
-    for (int j = 0; j < FN; j++) {
-        const int n = n0 + wn * TN + j * 16 + (lane & 15);
-        if (n >= N) continue;
-        const float b = bias ? bias[n] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * TM + i * 16 + 4 * (lane >> 4) + r;
-                if (m >= M) continue;
-                float v = acc[i][j][r] + b;
-                switch (act) {
-                case 1: v = act_relu(v); break;
-                case 2: v = act_gelu_tanh(v); break;
-                case 3: v = act_gelu_erf(v); break;
-                case 4: v = act_silu(v); break;
-                default: break;
-                }
-                float* o = out + (size_t)m * ldo + n;
-                *o = accumulate ? fmaf(alpha, v, *o) : v;
-            }
+// max over the N = 8 or 16 lanes that hold a row
+template <int N>
+__device__ __forceinline__ float lanes_max(float v) {
+    v = fmaxf(v, dpp_f32<0xb1, 0xf>(v, v));    // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp_f32<0x4e, 0xf>(v, v));    // quad_perm [2,3,0,1]
+    v = fmaxf(v, dpp_f32<0x141, 0xf>(v, v));   // row_half_mirror
+    return N == 8 ? v : fmaxf(v, dpp_f32<0x140, 0xf>(v, v));  // row_mirror
+}
+
+// The power of two that brings `mx` to [2^top, 2^(top + 1)), as its biased
+// exponent, kept where it and its inverse (254 minus it) are normal floats.
+__device__ __forceinline__ uint32_t scale_exp(float mx, int top) {
+    const int e = 254 + top - (int)((__float_as_uint(mx) >> 23) & 0xffu);
+    return (uint32_t)(e < 1 ? 1 : e > 253 ? 253 : e);
+}
+__device__ __forceinline__ float exp_float(uint32_t e) { return __uint_as_float(e << 23); }
+
+// Block barrier that orders LDS only: __syncthreads' release fence would also
+// wait for the global loads of the slab after next.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float act_of(float v, int act) {
+    switch (act) {
+    case 1: return act_relu(v);
+    case 2: return act_gelu_tanh(v);
+    case 3: return act_gelu_erf(v);
+    case 4: return act_silu(v);
+    default: return v;
     }
 }
 
-// The tiled form for M > 128 with 16-byte aligned rows (the conv GEMMs of
-// ACT's fp32 backbone and Octo's stems, the big fp32 projections): BM x BN
-// tiles, four waves in a 2 x 2 grid, 32-wide K slabs loaded as float4 runs
-// (coalesced 128-byte row segments) into registers while the previous slab
-// computes from the other LDS buffer. Within a 16-wide k chunk, lane group g
-// feeds k = 4g + t to the t-th of four MFMAs (the same order for A and B, so
-// each MFMA still sums matching products), which lets a lane read its four
-// A (or B) values as one ds_read_b128; LDS rows are padded to BK + 4 floats,
-// so the 16 rows one read touches fall on distinct banks.
+// The tiled form for M > 128 (the conv GEMMs of ACT's fp32 backbone and Octo's
+// stems, the fp32 projections) on the fp16 matrix cores: x W^T from the products
+// hh, hm and mh of the operands' two parts. Three v_mfma_f32_16x16x32_f16 take
+// 48 cycles of a SIMD where eight v_mfma_f32_16x16x4f32 take 256, and their
+// fp32 sums round once per 32 terms: against 64 bits the results are closer
+// (2-norm, N(0, 1) rows, K = 768: 3.6e-7 against 5.8e-7).
+//
+// Every row of x and of W has a scale of its own, a power of two taken out of
+// the sums exactly. It is guessed from the row's values in one slab (the first;
+// a convolution's centre tap, which always lies inside the image), so that they
+// reach 2^12, or from the tile's where the row has none; the maxima of all
+// slabs are kept, and a tile some row of which ends up outside [2^8, 2^15] is
+// computed once more with the scales of the true maxima. So no part overflows
+// and no operand loses more than 2^-33 of its row's largest value (2^-22 of
+// itself at worst). Infinities are left to plain fmaf chains.
+//
+// BM x BN tiles, four waves in a 2 x 2 grid. A K slab, KS steps of 32, is loaded as
+// float4 runs (whole 128-byte row segments per 8 lanes, 256 per 16 with KS = 2) into registers while
+// the slab before it computes, and split once per block on its way to LDS:
+// [part][k step][row][32 k] with the 16-byte chunks of a row permuted by its number, so
+// the 16 rows of one fragment read fall on distinct banks. The weights are the
+// first operand: a lane then holds four consecutive output columns.
 // CONV: x is an NHWC map and row m of A is output pixel m's k x k patch,
 // column (ky * k + kx) * Cin + ci (im2col's order), gathered by the A loads
-// themselves: with Cin % 32 == 0 a thread's float4 of a 32-wide slab always
-// lies in one tap, and its tap advances by 32 channels per slab. Same
+// themselves: with Cin % 32 == 0 a thread's float4 of a slab always lies in
+// one tap, and its tap advances by the slab's channels. Same
 // products in the same order as im2col + this kernel; no column matrix.
+// VEC: rows are 16-byte aligned runs; otherwise elements are loaded one by one.
 struct ConvGeom {
     int H, Wd, Cin, k, stride, pad, Wout;
 };
 
-template <int BM, int BN, bool CONV = false>
+template <int BM, int BN, int KS, bool CONV, bool VEC>
 __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out, int ldo,
                                                         const float* __restrict__ x, int ldx,
                                                         const float* __restrict__ W, int ldw,
                                                         const float* __restrict__ bias, int M, int N,
                                                         int K, int act, int accumulate, float alpha,
                                                         ConvGeom cg, float* __restrict__ part, int kchunk) {
-    constexpr int BK = 32, SP = BK + 4;
+    constexpr int BK = 32 * KS, LR = 8 * KS, ROWS = BM + BN;  // LR lanes hold a row of a slab
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
     constexpr int AV = BM * BK / 4 / 256, BV = BN * BK / 4 / 256;  // float4 loads per thread
     static_assert(AV >= 1 && BV >= 1 && TM % 16 == 0 && TN % 16 == 0, "tile");
-    __shared__ __attribute__((aligned(16))) float sm[2][(BM + BN) * SP];
+    __shared__ __attribute__((aligned(16))) char sm[2][2][KS][ROWS * 64];
+    __shared__ float unit[ROWS];  // what a row's sums are multiplied by in the end
+    __shared__ uint32_t guess[2];  // the tile's largest value of x and of W in the guess slab
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
@@ -139,14 +139,13 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
     const int kbeg = part ? blockIdx.z * kchunk : 0;
     if (part) K = K - kbeg < kchunk ? K - kbeg : kchunk;
 
-    // float4 v of a slab: row v / 8, k 4 (v % 8); rows past the matrix clamped
+    // float4 v of a slab: row v / LR, k 4 (v % LR); rows past the matrix clamped
     const float* ap[AV];
     const float* bp[BV];
-    int ao[AV], bo[BV], kk[AV > BV ? AV : BV];
     int iy0[AV], ix0[AV];  // CONV: the patch origin of each loaded row
 #pragma unroll
     for (int j = 0; j < AV; j++) {
-        const int v = tid + 256 * j, r = v >> 3, k = (v & 7) * 4;
+        const int v = tid + 256 * j, r = v / LR, k = (v % LR) * 4;
         const int m = m0 + r < M ? m0 + r : M - 1;
         if (CONV) {
             const int oy = m / cg.Wout, ox = m - oy * cg.Wout;
@@ -156,63 +155,92 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
         } else {
             ap[j] = x + (size_t)m * ldx + kbeg + k;
         }
-        ao[j] = r * SP + k;
     }
 #pragma unroll
     for (int j = 0; j < BV; j++) {
-        const int v = tid + 256 * j, r = v >> 3, k = (v & 7) * 4;
+        const int v = tid + 256 * j, r = v / LR, k = (v % LR) * 4;
         const int n = n0 + r < N ? n0 + r : N - 1;
         bp[j] = W + (size_t)n * ldw + kbeg + k;
-        bo[j] = (BM + r) * SP + k;
     }
-    const int kq = (tid & 7) * 4;  // this thread's k offset within a slab (same for every load)
-    (void)kk;
+    const int kq = (tid % LR) * 4;  // this thread's k offset within a slab (same for every load)
     float4 ra[AV], rb[BV];
     auto ld4 = [&](const float* p, int k) {
-        if (k + 4 <= K) return *reinterpret_cast<const float4*>(p);
+        if (VEC && k + 4 <= K) return *reinterpret_cast<const float4*>(p);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (k < K) v.x = p[0];
         if (k + 1 < K) v.y = p[1];
         if (k + 2 < K) v.z = p[2];
-        return v;  // k + 3 >= K here
+        if (k + 3 < K) v.w = p[3];
+        return v;
     };
     // CONV: the tap of this thread's next A slab (kbeg is a multiple of 32)
-    int ci = kq, kx = 0, ky = 0;
-    if (CONV && kbeg) {
-        const int t = kbeg / cg.Cin;
-        ci = kbeg - t * cg.Cin + kq;
+    int ci, kx, ky;
+    auto first_tap = [&] {
+        const int t = (kbeg + kq) / cg.Cin;
+        ci = kbeg + kq - t * cg.Cin;
         ky = t / cg.k;
         kx = t - ky * cg.k;
-    }
+    };
     auto gload = [&](int k0) {
+        const bool whole = VEC && k0 + BK <= K;  // wave-uniform: no lane meets the end of a row
         if (CONV) {  // called for k0 = 0, BK, 2 BK, ... in order
 #pragma unroll
             for (int j = 0; j < AV; j++) {
                 const int iy = iy0[j] + ky, ix = ix0[j] + kx;
                 ra[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd)
+                if (iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd && (KS == 1 || k0 + kq < K))
                     ra[j] = *reinterpret_cast<const float4*>(x + ((size_t)iy * cg.Wd + ix) * cg.Cin + ci);
             }
             ci += BK;
-            if (ci >= cg.Cin) {
+            while (ci >= cg.Cin) {  // (once, but for KS * 32 channels past a tap of 32)
                 ci -= cg.Cin;
                 if (++kx == cg.k) {
                     kx = 0;
                     ++ky;
                 }
             }
+        } else if (whole) {
+#pragma unroll
+            for (int j = 0; j < AV; j++) ra[j] = *reinterpret_cast<const float4*>(ap[j] + k0);
         } else {
 #pragma unroll
             for (int j = 0; j < AV; j++) ra[j] = ld4(ap[j] + k0, k0 + kq);
         }
+        if (whole) {
 #pragma unroll
-        for (int j = 0; j < BV; j++) rb[j] = ld4(bp[j] + k0, k0 + kq);
+            for (int j = 0; j < BV; j++) rb[j] = *reinterpret_cast<const float4*>(bp[j] + k0);
+        } else {
+#pragma unroll
+            for (int j = 0; j < BV; j++) rb[j] = ld4(bp[j] + k0, k0 + kq);
+        }
     };
+    float ma[AV], mb[BV];       // this thread's part of its rows' maxima
+    uint32_t ea[AV], eb[BV];    // the rows' scales (biased exponents)
+    // row r's 16-byte chunk q lies at chunk q ^ (-(r / 4) % 4): rows that share
+    // banks (4 apart) take different chunks, in the 16 lanes 0-3, 12-15, 20-23
+    // and 24-27 (and their like) that a ds_read_b128 serves at once
+    auto at = [](int r, int q) { return r * 64 + ((q ^ -(r >> 2)) & 3) * 16; };
     auto lstore = [&](int buf) {
+        const int ks = (tid % LR) >> 3, q = (tid & 7) >> 1, half = (tid & 1) * 8;
+        auto put = [&](int r, const float4& v, uint32_t e) {
+            const float s = exp_float(e);
+            uint2 h, m;
+            split2(v.x * s, v.y * s, h.x, m.x);
+            split2(v.z * s, v.w * s, h.y, m.y);
+            const int o = at(r, q) + half;
+            *reinterpret_cast<uint2*>(&sm[buf][0][ks][o]) = h;
+            *reinterpret_cast<uint2*>(&sm[buf][1][ks][o]) = m;
+        };
 #pragma unroll
-        for (int j = 0; j < AV; j++) *reinterpret_cast<float4*>(&sm[buf][ao[j]]) = ra[j];
+        for (int j = 0; j < AV; j++) {
+            ma[j] = absmax4(ma[j], ra[j]);
+            put((tid + 256 * j) / LR, ra[j], ea[j]);
+        }
 #pragma unroll
-        for (int j = 0; j < BV; j++) *reinterpret_cast<float4*>(&sm[buf][bo[j]]) = rb[j];
+        for (int j = 0; j < BV; j++) {
+            mb[j] = absmax4(mb[j], rb[j]);
+            put(BM + (tid + 256 * j) / LR, rb[j], eb[j]);
+        }
     };
 
     v4f acc[FM][FN];
@@ -220,83 +248,191 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
     for (int i = 0; i < FM; i++)
 #pragma unroll
         for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int r16 = lane & 15, g4 = (lane >> 4) * 4;
+    const int r16 = lane & 15, g = lane >> 4;
     auto compute = [&](int buf) {
-        const float* s = sm[buf];
 #pragma unroll
-        for (int kc = 0; kc < BK; kc += 16) {
-            float4 af[FM], bf[FN];
+        for (int ks = 0; ks < KS; ks++) {
+            f16x8 af[FM][2], bf[FN][2];
 #pragma unroll
-            for (int i = 0; i < FM; i++)
-                af[i] = *reinterpret_cast<const float4*>(s + (wm * TM + i * 16 + r16) * SP + kc + g4);
+            for (int p = 0; p < 2; p++) {
 #pragma unroll
-            for (int j = 0; j < FN; j++)
-                bf[j] = *reinterpret_cast<const float4*>(s + (BM + wn * TN + j * 16 + r16) * SP + kc + g4);
+                for (int i = 0; i < FM; i++)
+                    af[i][p] = *reinterpret_cast<const f16x8*>(&sm[buf][p][ks][at(wm * TM + i * 16 + r16, g)]);
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+                for (int j = 0; j < FN; j++)
+                    bf[j][p] = *reinterpret_cast<const f16x8*>(&sm[buf][p][ks][at(BM + wn * TN + j * 16 + r16, g)]);
+            }
+            auto mul = [&](int pa, int pb) {
 #pragma unroll
-                for (int j = 0; j < FN; j++) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i].x, bf[j].x, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i].y, bf[j].y, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i].z, bf[j].z, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i].w, bf[j].w, acc[i][j], 0, 0, 0);
-                }
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+                        acc[i][j] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j][pb], af[i][pa], acc[i][j], 0, 0, 0);
+            };
+            mul(0, 1);
+            mul(1, 0);
+            mul(0, 0);
         }
     };
 
-    const int nk = (K + BK - 1) / BK;
+    // the guess: rows' maxima in the first slab (CONV: x's from the centre tap)
+    if (tid < 2) guess[tid] = 0;
+    if (CONV) {
+        first_tap();
+#pragma unroll
+        for (int j = 0; j < AV; j++) {
+            const int iy = iy0[j] + cg.pad, ix = ix0[j] + cg.pad;
+            const bool in = iy < cg.H && ix < cg.Wd;  // (not with a kernel reaching past the far border only)
+            ma[j] = absmax4(0.0f, in ? *reinterpret_cast<const float4*>(x + ((size_t)iy * cg.Wd + ix) * cg.Cin + kq)
+                                     : make_float4(0.f, 0.f, 0.f, 0.f));
+        }
+    }
     gload(0);
-    lstore(0);
-    if (nk > 1) gload(BK);
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        compute(buf);
-        if (kt + 1 < nk) {
-            lstore(buf ^ 1);  // slab kt + 1, loaded during this compute
-            if (kt + 2 < nk) gload((kt + 2) * BK);
+#pragma unroll
+    for (int j = 0; j < AV; j++) ma[j] = lanes_max<LR>(CONV ? ma[j] : absmax4(0.0f, ra[j]));
+#pragma unroll
+    for (int j = 0; j < BV; j++) mb[j] = lanes_max<LR>(absmax4(0.0f, rb[j]));
+    bool none = false;  // a row without values in the guess slab takes the tile's guess
+#pragma unroll
+    for (int j = 0; j < AV; j++) none = none || ma[j] == 0.0f;
+#pragma unroll
+    for (int j = 0; j < BV; j++) none = none || mb[j] == 0.0f;
+    if (__syncthreads_or(none)) {
+        float ta = 0.0f, tb = 0.0f;
+#pragma unroll
+        for (int j = 0; j < AV; j++) ta = fmaxf(ta, ma[j]);
+#pragma unroll
+        for (int j = 0; j < BV; j++) tb = fmaxf(tb, mb[j]);
+        ta = wave_max_f32(ta);
+        tb = wave_max_f32(tb);
+        if (lane == 0) {  // floats >= 0 order as their bits
+            atomicMax(&guess[0], __float_as_uint(ta));
+            atomicMax(&guess[1], __float_as_uint(tb));
         }
         __syncthreads();
+#pragma unroll
+        for (int j = 0; j < AV; j++) ma[j] = ma[j] > 0.0f ? ma[j] : __uint_as_float(guess[0]);
+#pragma unroll
+        for (int j = 0; j < BV; j++) mb[j] = mb[j] > 0.0f ? mb[j] : __uint_as_float(guess[1]);
     }
+#pragma unroll
+    for (int j = 0; j < AV; j++) ea[j] = scale_exp(ma[j], 12);
+#pragma unroll
+    for (int j = 0; j < BV; j++) eb[j] = scale_exp(mb[j], 12);
 
-    if (part) {
-        float* pz = part + (size_t)blockIdx.z * M * N;
+    const int nk = (K + BK - 1) / BK;
+    bool again = false, bad;
+    for (;;) {
 #pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int n = n0 + wn * TN + j * 16 + r16;
-            if (n >= N) continue;
+        for (int j = 0; j < AV; j++) ma[j] = 0.0f;
 #pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int m = m0 + wm * TM + i * 16 + g4 + r;
-                    if (m < M) pz[(size_t)m * N + n] = acc[i][j][r];
-                }
+        for (int j = 0; j < BV; j++) mb[j] = 0.0f;
+        lstore(0);
+        if (nk > 1) gload(BK);
+        lds_barrier();
+        for (int kt = 0; kt < nk; kt++) {
+            const int buf = kt & 1;
+            compute(buf);
+            if (kt + 1 < nk) {
+                lstore(buf ^ 1);  // slab kt + 1, loaded during this compute
+                if (kt + 2 < nk) gload((kt + 2) * BK);
+            }
+            lds_barrier();
         }
-        return;
-    }
+        // the rows' true maxima under the scales used; what the sums are
+        // multiplied by, for the epilogue
+        bool off = false, inf = false;
+        auto check = [&](float& mx, uint32_t e, int r) {
+            mx = lanes_max<LR>(mx);
+            const float t = mx * exp_float(e);
+            off = off || !(mx == 0.0f || (t >= 256.0f && t <= 32768.0f));
+            inf = inf || !(mx <= 3.4028235e38f);
+            if (tid % LR == 0) unit[r] = exp_float(254u - e);
+        };
 #pragma unroll
-    for (int j = 0; j < FN; j++) {
-        const int n = n0 + wn * TN + j * 16 + r16;
-        if (n >= N) continue;
-        const float b = bias ? bias[n] : 0.0f;
+        for (int j = 0; j < AV; j++) check(ma[j], ea[j], (tid + 256 * j) / LR);
+#pragma unroll
+        for (int j = 0; j < BV; j++) check(mb[j], eb[j], BM + (tid + 256 * j) / LR);
+        // a second pass can only find values that are not finite, or rows so
+        // small that 2^126 leaves them below 2^8
+        bad = __syncthreads_or(again ? inf : off);
+        if (!bad || again) break;
+        again = true;
+#pragma unroll
+        for (int j = 0; j < AV; j++) ea[j] = scale_exp(ma[j], 14);
+#pragma unroll
+        for (int j = 0; j < BV; j++) eb[j] = scale_exp(mb[j], 14);
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * TM + i * 16 + g4 + r;
-                if (m >= M) continue;
-                float v = acc[i][j][r] + b;
-                switch (act) {
-                case 1: v = act_relu(v); break;
-                case 2: v = act_gelu_tanh(v); break;
-                case 3: v = act_gelu_erf(v); break;
-                case 4: v = act_silu(v); break;
-                default: break;
+            for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (CONV) first_tap();
+        gload(0);
+    }
+
+    float* dst = part ? part + (size_t)blockIdx.z * M * N : out;
+    const int ldd = part ? N : ldo;
+    if (bad) {  // one fmaf chain per output; its speed does not matter
+        for (int e = tid; e < BM * BN; e += 256) {
+            const int m = m0 + e / BN, n = n0 + e % BN;
+            if (m >= M || n >= N) continue;
+            const float* wr = W + (size_t)n * ldw + kbeg;
+            float v = 0.0f;
+            if (CONV) {
+                const int oy = m / cg.Wout, ox = m - oy * cg.Wout;
+                for (int k = 0; k < K; k++) {
+                    const int t = (kbeg + k) / cg.Cin, c = kbeg + k - t * cg.Cin;
+                    const int iy = oy * cg.stride - cg.pad + t / cg.k, ix = ox * cg.stride - cg.pad + t % cg.k;
+                    const bool in = iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd;
+                    v = fmaf(in ? x[((size_t)iy * cg.Wd + ix) * cg.Cin + c] : 0.0f, wr[k], v);
                 }
-                float* o = out + (size_t)m * ldo + n;
-                *o = accumulate ? fmaf(alpha, v, *o) : v;
+            } else {
+                const float* xr = x + (size_t)m * ldx + kbeg;
+                for (int k = 0; k < K; k++) v = fmaf(xr[k], wr[k], v);
             }
+            float* o = dst + (size_t)m * ldd + n;
+            if (!part) v = act_of(v + (bias ? bias[n] : 0.0f), act);
+            *o = !part && accumulate ? fmaf(alpha, v, *o) : v;
+        }
+        return;
+    }
+
+    // lane: row m = r16 of a fragment, columns n = 4 g .. 4 g + 3
+    const bool vec = (ldd & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+        const int n = n0 + wn * TN + j * 16 + 4 * g;
+        if (n >= N) continue;
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias && !part)
+            for (int r = 0; r < 4; r++)
+                if (n + r < N) b[r] = bias[n + r];
+#pragma unroll
+        for (int i = 0; i < FM; i++) {
+            const int m = m0 + wm * TM + i * 16 + r16;
+            if (m >= M) continue;
+            float* o = dst + (size_t)m * ldd + n;
+            const float ua = unit[wm * TM + i * 16 + r16];
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[r] = acc[i][j][r] * (ua * unit[BM + wn * TN + j * 16 + 4 * g + r]);
+                if (!part) v[r] = act_of(v[r] + b[r], act);
+            }
+            if (vec && n + 4 <= N) {
+                if (!part && accumulate) {
+                    const float4 d = *reinterpret_cast<const float4*>(o);
+                    v[0] = fmaf(alpha, v[0], d.x);
+                    v[1] = fmaf(alpha, v[1], d.y);
+                    v[2] = fmaf(alpha, v[2], d.z);
+                    v[3] = fmaf(alpha, v[3], d.w);
+                }
+                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+                for (int r = 0; r < 4 && n + r < N; r++) o[r] = !part && accumulate ? fmaf(alpha, v[r], o[r]) : v[r];
+            }
+        }
     }
 }
 
@@ -379,14 +515,7 @@ __global__ __launch_bounds__(W * 64) void linear_f32_skinny(float* __restrict__ 
         const int l = e & 63, r = (e >> 6) & 3, i = e >> 8;
         const int m = mb + 16 * i + 4 * (l >> 4) + r, nn = n0 + (l & 15);
         if (m >= M || nn >= N) continue;
-        v = v + (bias ? bias[nn] : 0.0f);
-        switch (act) {
-        case 1: v = act_relu(v); break;
-        case 2: v = act_gelu_tanh(v); break;
-        case 3: v = act_gelu_erf(v); break;
-        case 4: v = act_silu(v); break;
-        default: break;
-        }
+        v = act_of(v + (bias ? bias[nn] : 0.0f), act);
         float* o = out + (size_t)m * ldo + nn;
         *o = accumulate ? fmaf(alpha, v, *o) : v;
     }
@@ -441,14 +570,7 @@ __global__ __launch_bounds__(256) void linear_f32_split_reduce(float* __restrict
         float v = part[e];
         for (int z = 1; z < S; z++) v += part[z * MN + e];
         const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
-        v = v + (bias ? bias[n] : 0.0f);
-        switch (act) {
-        case 1: v = act_relu(v); break;
-        case 2: v = act_gelu_tanh(v); break;
-        case 3: v = act_gelu_erf(v); break;
-        case 4: v = act_silu(v); break;
-        default: break;
-        }
+        v = act_of(v + (bias ? bias[n] : 0.0f), act);
         float* o = out + (size_t)m * ldo + n;
         *o = accumulate ? fmaf(alpha, v, *o) : v;
     }
@@ -456,19 +578,25 @@ __global__ __launch_bounds__(256) void linear_f32_split_reduce(float* __restrict
 
 constexpr int kCUs = 256;  // MI355X compute units
 
+struct F32Call {
+    float* out;
+    int ldo;
+    const float* x;
+    int ldx;
+    const float* W;
+    int ldw;
+    const float* bias;
+    int M, N, K, act, accumulate;
+    float alpha;
+    ConvGeom cg;
+};
+
 // Split-K plan for M > 128 over K >= 1024 when 64 x 64 tiles number < 128
 // (ResNet's last stages): S chunks of K (multiples of 32, >= 256) so that
 // S x tiles reaches about two blocks per CU, S <= 8.
 struct F32Split {
     int S = 1, kchunk = 0;
 };
-// VLA_HIP_F32_SMALL_TILES=0 keeps 64 x 64 tiles for few-tile fp32 layers
-// (read per call; A/B runs)
-static bool f32_small_tiles_on() {
-    const char* e = std::getenv("VLA_HIP_F32_SMALL_TILES");
-    return !(e && e[0] == '0' && e[1] == '\0');
-}
-
 F32Split f32_split_plan(int M, int N, int K) {
     F32Split p;
     const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
@@ -483,27 +611,42 @@ F32Split f32_split_plan(int M, int N, int K) {
     return p;
 }
 
-void launch_f32_split(float* out, int ldo, const float* x, int ldx, const float* W, int ldw, const float* bias,
-                      int M, int N, int K, int act, int accumulate, float alpha, const ConvGeom& cg, bool conv,
-                      const F32Split& p, float* part, hipStream_t st) {
-    const dim3 grid((N + 63) / 64, (M + 63) / 64, p.S);
-    if (conv)
-        linear_f32_tiled<64, 64, true><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, 0, 0, 1.0f, cg,
-                                                             part, p.kchunk);
-    else
-        linear_f32_tiled<64, 64><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, 0, 0, 1.0f, cg, part,
-                                                       p.kchunk);
-    VLA_LAUNCH_CHECK();
-    const int64_t MN = (int64_t)M * N;
-    const int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
-    linear_f32_split_reduce<<<blocks, 256, 0, st>>>(out, ldo, part, p.S, M, N, bias, act, accumulate, alpha);
+template <int BM, int BN, int KS, bool CONV, bool VEC>
+void launch_tile(const F32Call& c, float* part, int S, int kchunk, hipStream_t st) {
+    const dim3 grid((c.N + BN - 1) / BN, (c.M + BM - 1) / BM, S);
+    linear_f32_tiled<BM, BN, KS, CONV, VEC><<<grid, 256, 0, st>>>(c.out, c.ldo, c.x, c.ldx, c.W, c.ldw, c.bias, c.M, c.N,
+                                                              c.K, c.act, c.accumulate, c.alpha, c.cg, part, kchunk);
     VLA_LAUNCH_CHECK();
 }
 
-// VLA_F32_TILED=0 keeps the LDS-scalar kernel (A/B comparisons)
-bool env_off_f32tiled() {
-    const char* e = std::getenv("VLA_F32_TILED");
-    return e && e[0] == '0' && e[1] == '\0';
+// The largest tile that still gives the CUs enough blocks: one block's slabs
+// are a serial chain of LDS round trips, splitting and products, and two or
+// three blocks on a CU fill each other's gaps. The smallest tile takes 64-wide
+// slabs, half the round trips (177 x 960 x 960 17.5 -> 13.1 us); on the larger
+// ones the second step costs residency (690 x 768 x 3072 on 64 x 64 29.0 ->
+// 39.6). Measured, us (fp32 matrix cores | 32 x 32, 64 x 64, 128 x 64):
+// 690 x 768 x 3072 64.5 | 43.7 27.5 32; 1024 x 768 x 3072 64.1 | 50.4 29.9 34;
+// 2048 x 2048 x 2048 156 | 147 87.0 76.9; 19200 x 576 x 64 29.2 | 23.5 18.8 23;
+// 4800 x 1152 x 128 33.3 | 21.2 26.9 34; 690 x 768 x 768 23.8 | 14.0 19.8 26.
+template <bool CONV, bool VEC>
+void launch_tiles(const F32Call& c, hipStream_t st) {
+    auto blocks = [&](int bm, int bn) { return (long)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn); };
+    if (blocks(128, 64) >= 2 * kCUs) launch_tile<128, 64, 1, CONV, VEC>(c, nullptr, 1, 0, st);
+    else if (blocks(64, 64) >= kCUs) launch_tile<64, 64, 1, CONV, VEC>(c, nullptr, 1, 0, st);
+    else launch_tile<32, 32, 2, CONV, VEC>(c, nullptr, 1, 0, st);
+}
+
+// Shapes whose 32 x 32 tiles leave CUs idle while each walks a long K.
+bool few_tiles(int M, int N, int K) { return K >= 1024 && (long)((M + 31) / 32) * ((N + 31) / 32) < kCUs; }
+
+void launch_f32_split(const F32Call& c, bool conv, const F32Split& p, float* part, hipStream_t st) {
+    if (conv) launch_tile<64, 64, 1, true, true>(c, part, p.S, p.kchunk, st);
+    else launch_tile<64, 64, 1, false, true>(c, part, p.S, p.kchunk, st);
+    const int64_t MN = (int64_t)c.M * c.N;
+    const int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
+    linear_f32_split_reduce<<<blocks, 256, 0, st>>>(c.out, c.ldo, part, p.S, c.M, c.N, c.bias, c.act, c.accumulate,
+                                                    c.alpha);
+    VLA_LAUNCH_CHECK();
 }
 
 }  // namespace
@@ -529,58 +672,31 @@ void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float
         VLA_LAUNCH_CHECK();
         return;
     }
-    if (ldx % 4 == 0 && ldw % 4 == 0 && aligned(x, 16) && aligned(W, 16) && !env_off_f32tiled()) {
-        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
-        const F32Split sp = f32_split_plan(M, N, K);
-        if (sp.S > 1 && work && work_floats >= (size_t)sp.S * M * N && aligned(work, 16)) {
-            // few tiles over a long K with a workspace: 64 x 64 tiles split over K
-            launch_f32_split(out, ldo, x, ldx, W, ldw, bias, M, N, K, act, accumulate, alpha, ConvGeom{}, false, sp,
-                             work, st);
-            return;
-        }
-        if (t64 < 128 && K >= 1024) {
-            // few tiles over a long K (ResNet's last stages): the split-K form,
-            // 64-row x 16-column blocks whose 8 waves share K, so the chain of
-            // dependent loads per wave is an eighth of K
-            const dim3 grid((N + 15) / 16, (M + 63) / 64);
-            linear_f32_skinny<4, 8, true><<<grid, 512, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                                 accumulate, alpha);
-            VLA_LAUNCH_CHECK();
-            return;
-        }
-        // 128 x 64 tiles when they still give every CU work, 64 x 64 from 128
-        // such tiles, else 32 x 32 (a fourth of the fp32 matrix work per
-        // block: Octo's 256 x 768 x 512 token projections, 48 tiles of 64 x
-        // 64, were ~20 us each, one fp32 MFMA chain of a whole tile per CU)
-        const long t128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-        if (t128 >= 256) {
-            const dim3 grid((N + 63) / 64, (M + 127) / 128);
-            linear_f32_tiled<128, 64><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                            accumulate, alpha, ConvGeom{}, nullptr, 0);
-        } else if (t64 < 128 && f32_small_tiles_on()) {
-            const dim3 grid((N + 31) / 32, (M + 31) / 32);
-            linear_f32_tiled<32, 32><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                           accumulate, alpha, ConvGeom{}, nullptr, 0);
-        } else {
-            const dim3 grid((N + 63) / 64, (M + 63) / 64);
-            linear_f32_tiled<64, 64><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                           accumulate, alpha, ConvGeom{}, nullptr, 0);
-        }
+    const F32Call c{out, ldo, x, ldx, W, ldw, bias, M, N, K, act, accumulate, alpha, ConvGeom{}};
+    const bool vec = ldx % 4 == 0 && ldw % 4 == 0 && aligned(x, 16) && aligned(W, 16);
+    if (!vec) {
+        launch_tiles<false, false>(c, st);
+        return;
+    }
+    const F32Split sp = f32_split_plan(M, N, K);
+    if (sp.S > 1 && work && work_floats >= (size_t)sp.S * M * N && aligned(work, 16)) {
+        // few tiles over a long K with a workspace: 64 x 64 tiles split over K
+        launch_f32_split(c, false, sp, work, st);
+        return;
+    }
+    if (few_tiles(M, N, K)) {
+        // few tiles over a long K (ResNet's last stages): the split-K form,
+        // 64-row x 16-column blocks whose 8 waves share K, so the chain of
+        // dependent loads per wave is an eighth of K (300 x 4608 x 512 48 us
+        // against 64, 302 x 3200 x 512 35 against 46; with 304 tiles of 32 x
+        // 32 the tiles are ahead: 1200 x 2304 x 256 36 against 49)
+        const dim3 grid((N + 15) / 16, (M + 63) / 64);
+        linear_f32_skinny<4, 8, true><<<grid, 512, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
+                                                             accumulate, alpha);
         VLA_LAUNCH_CHECK();
         return;
     }
-    // small grids take 32 x 32 tiles so more CUs get work
-    const long big = (long)((M + 63) / 64) * ((N + 63) / 64);
-    if (big >= 128) {
-        const dim3 grid((N + 63) / 64, (M + 63) / 64);
-        linear_f32_kernel<64, 64><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                        accumulate, alpha);
-    } else {
-        const dim3 grid((N + 31) / 32, (M + 31) / 32);
-        linear_f32_kernel<32, 32><<<grid, 256, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
-                                                        accumulate, alpha);
-    }
-    VLA_LAUNCH_CHECK();
+    launch_tiles<false, true>(c, st);
 }
 
 bool launch_conv_f32_implicit(float* out, const float* x, int H, int Wd, int Cin, int k, int stride, int pad,
@@ -597,29 +713,19 @@ bool launch_conv_f32_implicit(float* out, const float* x, int H, int Wd, int Cin
                     (int64_t)(Wout - 1) * stride + k <= (int64_t)Wd + 2 * pad,
                 "conv_f32: output larger than the padded input allows");
     if (Cin % 32 || K64 > INT32_MAX || M64 > INT32_MAX || (int64_t)H * Wd * Cin > INT32_MAX) return false;
-    if (!aligned(x, 16) || !aligned(W, 16) || env_off_f32tiled()) return false;
+    if (!aligned(x, 16) || !aligned(W, 16)) return false;
     const int M = (int)M64, K = (int)K64, N = Cout;
     if (M <= 128) return false;
-    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     const ConvGeom cg{H, Wd, Cin, k, stride, pad, Wout};
     const F32Split sp = f32_split_plan(M, N, K);
+    const F32Call c{out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg};
     if (sp.S > 1) {  // as launch_linear_f32: split over K with a workspace, else not here
         if (!(work && work_floats >= (size_t)sp.S * M * N && aligned(work, 16))) return false;
-        launch_f32_split(out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg, true, sp, work, st);
+        launch_f32_split(c, true, sp, work, st);
         return true;
     }
-    if (t64 < 128 && K >= 1024) return false;  // the skinny route of launch_linear_f32
-    const long t128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-    if (t128 >= 256) {
-        const dim3 grid((N + 63) / 64, (M + 127) / 128);
-        linear_f32_tiled<128, 64, true><<<grid, 256, 0, st>>>(out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg,
-                                                              nullptr, 0);
-    } else {
-        const dim3 grid((N + 63) / 64, (M + 63) / 64);
-        linear_f32_tiled<64, 64, true><<<grid, 256, 0, st>>>(out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg,
-                                                             nullptr, 0);
-    }
-    VLA_LAUNCH_CHECK();
+    if (few_tiles(M, N, K)) return false;  // the skinny route of launch_linear_f32
+    launch_tiles<true, true>(c, st);
     return true;
 }
 
