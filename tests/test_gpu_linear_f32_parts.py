@@ -29,7 +29,8 @@ def data(M, K, N, seed=0):
 
 @pytest.mark.parametrize("M,K,N", [
     (129, 32, 32), (129, 33, 33), (160, 64, 40), (177, 960, 96), (511, 96, 510), (512, 100, 512),     # 32 x 32
-    (1024, 160, 1024), (1025, 161, 1023), (1030, 100, 1030),                                         # 64 x 64
+    (1024, 160, 1024), (1025, 161, 1023), (1030, 100, 1030), (1024, 32, 1000), (700, 65, 768),       # 64 x 64, two groups
+    (2500, 70, 1024), (2500, 96, 830),                                                               # 64 x 64
     (4096, 70, 1024), (4100, 64, 1030),                                                              # 128 x 64
     (300, 1100, 400), (1200, 1100, 260),                                                             # few tiles, long K
 ])

@@ -113,12 +113,16 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // one tap, and its tap advances by the slab's channels. Same
 // products in the same order as im2col + this kernel; no column matrix.
 // VEC: rows are 16-byte aligned runs; otherwise elements are loaded one by one.
+// G = 2: two groups of four waves take half of the block's K slabs each, with
+// slabs, scales and sums of their own; the sums meet in LDS and each group
+// finishes half of the tile. Twice the waves where the tiles alone leave a CU
+// one block (4800 x 1152 x 128 21.6 -> 18.3 us).
 struct ConvGeom {
     int H, Wd, Cin, k, stride, pad, Wout;
 };
 
-template <int BM, int BN, int KS, bool CONV, bool VEC>
-__global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out, int ldo,
+template <int BM, int BN, int KS, int G, bool CONV, bool VEC>
+__global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ out, int ldo,
                                                         const float* __restrict__ x, int ldx,
                                                         const float* __restrict__ W, int ldw,
                                                         const float* __restrict__ bias, int M, int N,
@@ -127,17 +131,25 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
     constexpr int BK = 32 * KS, LR = 8 * KS, ROWS = BM + BN;  // LR lanes hold a row of a slab
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
     constexpr int AV = BM * BK / 4 / 256, BV = BN * BK / 4 / 256;  // float4 loads per thread
-    static_assert(AV >= 1 && BV >= 1 && TM % 16 == 0 && TN % 16 == 0, "tile");
-    __shared__ __attribute__((aligned(16))) char sm[2][2][KS][ROWS * 64];
-    __shared__ float unit[ROWS];  // what a row's sums are multiplied by in the end
-    __shared__ uint32_t guess[2];  // the tile's largest value of x and of W in the guess slab
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    static_assert(AV >= 1 && BV >= 1 && TM % 16 == 0 && TN % 16 == 0 && FM % G == 0, "tile");
+    __shared__ __attribute__((aligned(16))) char smem[G][2][2][KS][ROWS * 64];
+    __shared__ float units[G][ROWS];  // what a row's sums are multiplied by in the end
+    __shared__ uint32_t guesses[G][2];  // the tile's largest value of x and of W in the guess slab
+    const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    auto& sm = smem[grp];
+    auto& unit = units[grp];
+    auto& guess = guesses[grp];
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     // split K (part != null): chunk blockIdx.z of kchunk columns, raw sums into
     // its slice of part; K becomes the chunk's length
-    const int kbeg = part ? blockIdx.z * kchunk : 0;
-    if (part) K = K - kbeg < kchunk ? K - kbeg : kchunk;
+    const int kblk = part ? blockIdx.z * kchunk : 0;
+    if (part) K = K - kblk < kchunk ? K - kblk : kchunk;
+    const int kall = K;  // the block's columns; from here on kbeg, K: the group's
+    const int nk = ((K + BK - 1) / BK + G - 1) / G;
+    const int kbeg = G > 1 ? kblk + grp * nk * BK : kblk;
+    if constexpr (G > 1) K = K - grp * nk * BK < nk * BK ? K - grp * nk * BK : nk * BK;  // (0 or less: no columns)
 
     // float4 v of a slab: row v / LR, k 4 (v % LR); rows past the matrix clamped
     const float* ap[AV];
@@ -188,7 +200,7 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
             for (int j = 0; j < AV; j++) {
                 const int iy = iy0[j] + ky, ix = ix0[j] + kx;
                 ra[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd && (KS == 1 || k0 + kq < K))
+                if (iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd && ((KS == 1 && G == 1) || k0 + kq < K))
                     ra[j] = *reinterpret_cast<const float4*>(x + ((size_t)iy * cg.Wd + ix) * cg.Cin + ci);
             }
             ci += BK;
@@ -321,7 +333,6 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
 #pragma unroll
     for (int j = 0; j < BV; j++) eb[j] = scale_exp(mb[j], 12);
 
-    const int nk = (K + BK - 1) / BK;
     bool again = false, bad;
     for (;;) {
 #pragma unroll
@@ -374,28 +385,57 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
     float* dst = part ? part + (size_t)blockIdx.z * M * N : out;
     const int ldd = part ? N : ldo;
     if (bad) {  // one fmaf chain per output; its speed does not matter
-        for (int e = tid; e < BM * BN; e += 256) {
+        for (int e = threadIdx.x; e < BM * BN; e += 256 * G) {
             const int m = m0 + e / BN, n = n0 + e % BN;
             if (m >= M || n >= N) continue;
-            const float* wr = W + (size_t)n * ldw + kbeg;
+            const float* wr = W + (size_t)n * ldw + kblk;
             float v = 0.0f;
             if (CONV) {
                 const int oy = m / cg.Wout, ox = m - oy * cg.Wout;
-                for (int k = 0; k < K; k++) {
-                    const int t = (kbeg + k) / cg.Cin, c = kbeg + k - t * cg.Cin;
+                for (int k = 0; k < kall; k++) {
+                    const int t = (kblk + k) / cg.Cin, c = kblk + k - t * cg.Cin;
                     const int iy = oy * cg.stride - cg.pad + t / cg.k, ix = ox * cg.stride - cg.pad + t % cg.k;
                     const bool in = iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd;
                     v = fmaf(in ? x[((size_t)iy * cg.Wd + ix) * cg.Cin + c] : 0.0f, wr[k], v);
                 }
             } else {
-                const float* xr = x + (size_t)m * ldx + kbeg;
-                for (int k = 0; k < K; k++) v = fmaf(xr[k], wr[k], v);
+                const float* xr = x + (size_t)m * ldx + kblk;
+                for (int k = 0; k < kall; k++) v = fmaf(xr[k], wr[k], v);
             }
             float* o = dst + (size_t)m * ldd + n;
             if (!part) v = act_of(v + (bias ? bias[n] : 0.0f), act);
             *o = !part && accumulate ? fmaf(alpha, v, *o) : v;
         }
         return;
+    }
+
+    // the groups' sums of the tile: group g finishes fragment rows g FM / G ..
+    constexpr int FG = FM / G;
+    if constexpr (G == 2) {
+        // (the barrier of `bad` lies after the last read of the slabs)
+        v4f* mine = reinterpret_cast<v4f*>(&smem[grp][0][0][0][0]) + tid;
+        const v4f* other = reinterpret_cast<const v4f*>(&smem[grp ^ 1][0][0][0][0]) + tid;
+#pragma unroll
+        for (int i = 0; i < FG; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                v4f v = grp ? acc[i][j] : acc[FG + i][j];  // the other group's half
+                const float ua = unit[wm * TM + (grp ? i : FG + i) * 16 + r16];
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] *= ua * unit[BM + wn * TN + j * 16 + 4 * g + r];
+                mine[(i * FN + j) * 256] = v;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < FG; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                v4f v = grp ? acc[FG + i][j] : acc[i][j];
+                const float ua = unit[wm * TM + (grp ? FG + i : i) * 16 + r16];
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] *= ua * unit[BM + wn * TN + j * 16 + 4 * g + r];
+                acc[i][j] = v + other[(i * FN + j) * 256];
+            }
     }
 
     // lane: row m = r16 of a fragment, columns n = 4 g .. 4 g + 3
@@ -409,15 +449,15 @@ __global__ __launch_bounds__(256) void linear_f32_tiled(float* __restrict__ out,
             for (int r = 0; r < 4; r++)
                 if (n + r < N) b[r] = bias[n + r];
 #pragma unroll
-        for (int i = 0; i < FM; i++) {
-            const int m = m0 + wm * TM + i * 16 + r16;
+        for (int i = 0; i < FG; i++) {
+            const int fr = wm * TM + (grp * FG + i) * 16 + r16, m = m0 + fr;
             if (m >= M) continue;
             float* o = dst + (size_t)m * ldd + n;
-            const float ua = unit[wm * TM + i * 16 + r16];
+            const float ua = unit[fr];
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                v[r] = acc[i][j][r] * (ua * unit[BM + wn * TN + j * 16 + 4 * g + r]);
+                v[r] = G > 1 ? acc[i][j][r] : acc[i][j][r] * (ua * unit[BM + wn * TN + j * 16 + 4 * g + r]);
                 if (!part) v[r] = act_of(v[r] + b[r], act);
             }
             if (vec && n + 4 <= N) {
@@ -627,37 +667,42 @@ F32Split f32_split_plan(int M, int N, int K) {
     return p;
 }
 
-template <int BM, int BN, int KS, bool CONV, bool VEC>
+template <int BM, int BN, int KS, int G, bool CONV, bool VEC>
 void launch_tile(const F32Call& c, float* part, int S, int kchunk, hipStream_t st) {
     const dim3 grid((c.N + BN - 1) / BN, (c.M + BM - 1) / BM, S);
-    linear_f32_tiled<BM, BN, KS, CONV, VEC><<<grid, 256, 0, st>>>(c.out, c.ldo, c.x, c.ldx, c.W, c.ldw, c.bias, c.M, c.N,
+    linear_f32_tiled<BM, BN, KS, G, CONV, VEC><<<grid, 256 * G, 0, st>>>(c.out, c.ldo, c.x, c.ldx, c.W, c.ldw, c.bias, c.M, c.N,
                                                               c.K, c.act, c.accumulate, c.alpha, c.cg, part, kchunk);
     VLA_LAUNCH_CHECK();
 }
 
-// The largest tile that still gives the CUs enough blocks: one block's slabs
-// are a serial chain of LDS round trips, splitting and products, and two or
-// three blocks on a CU fill each other's gaps. The smallest tile takes 64-wide
-// slabs, half the round trips (177 x 960 x 960 17.5 -> 13.1 us); on the larger
-// ones the second step costs residency (690 x 768 x 3072 on 64 x 64 29.0 ->
-// 39.6). Measured, us (fp32 matrix cores | 32 x 32, 64 x 64, 128 x 64):
-// 690 x 768 x 3072 64.5 | 43.7 27.5 32; 1024 x 768 x 3072 64.1 | 50.4 29.9 34;
-// 2048 x 2048 x 2048 156 | 147 87.0 76.9; 19200 x 576 x 64 29.2 | 23.5 18.8 23;
-// 4800 x 1152 x 128 33.3 | 21.2 26.9 34; 690 x 768 x 768 23.8 | 14.0 19.8 26.
+// The largest tile that still gives the CUs enough waves: a group's slabs are a
+// serial chain of LDS round trips, splitting and products, and two or three
+// groups on a CU fill each other's gaps. From two blocks of 64 x 64 per CU those
+// are blocks; from half a block per CU, two groups of one block that share its
+// K; below, 32 x 32 tiles, with 64-wide slabs, half the round trips (177 x 960 x
+// 960 17.5 -> 13.1 us); on the larger ones the second step costs residency (690
+// x 768 x 3072 on 64 x 64 29.0 -> 39.6). Measured, us (fp32 matrix cores | 32 x
+// 32, 64 x 64, 64 x 64 by two groups, 128 x 64):
+// 690 x 768 x 3072 64.5 | 39.3 28.6 30.8 32; 1024 x 768 x 3072 64.1 | 49.3 30.9 33.6 34;
+// 2048 x 2048 x 2048 156 | 140 89.8 90.6 80.7; 19200 x 576 x 64 29.2 | 22.8 19.2 17.5 23;
+// 4800 x 1152 x 128 33.3 | 21.4 26.2 18.3 34; 690 x 768 x 768 23.8 | 14.2 19.4 13.9 26;
+// 690 x 3072 x 768 78 | 42.6 57.2 37.0; 302 x 512 x 3200 18.8 | 14.7 16.0 12.5;
+// 256 x 768 x 512 (32 blocks of 64 x 64) 9.6 | 8.9 16.2 12.3; 177 x 960 x 960 (45) 14.3 | 13.0 21.9 15.2.
 template <bool CONV, bool VEC>
 void launch_tiles(const F32Call& c, hipStream_t st) {
     auto blocks = [&](int bm, int bn) { return (long)((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn); };
-    if (blocks(128, 64) >= 2 * kCUs) launch_tile<128, 64, 1, CONV, VEC>(c, nullptr, 1, 0, st);
-    else if (blocks(64, 64) >= kCUs) launch_tile<64, 64, 1, CONV, VEC>(c, nullptr, 1, 0, st);
-    else launch_tile<32, 32, 2, CONV, VEC>(c, nullptr, 1, 0, st);
+    if (blocks(128, 64) >= 2 * kCUs) launch_tile<128, 64, 1, 1, CONV, VEC>(c, nullptr, 1, 0, st);
+    else if (blocks(64, 64) >= 2 * kCUs) launch_tile<64, 64, 1, 1, CONV, VEC>(c, nullptr, 1, 0, st);
+    else if (2 * blocks(64, 64) >= kCUs) launch_tile<64, 64, 1, 2, CONV, VEC>(c, nullptr, 1, 0, st);
+    else launch_tile<32, 32, 2, 1, CONV, VEC>(c, nullptr, 1, 0, st);
 }
 
 // Shapes whose 32 x 32 tiles leave CUs idle while each walks a long K.
 bool few_tiles(int M, int N, int K) { return K >= 1024 && (long)((M + 31) / 32) * ((N + 31) / 32) < kCUs; }
 
 void launch_f32_split(const F32Call& c, bool conv, const F32Split& p, float* part, hipStream_t st) {
-    if (conv) launch_tile<64, 64, 1, true, true>(c, part, p.S, p.kchunk, st);
-    else launch_tile<64, 64, 1, false, true>(c, part, p.S, p.kchunk, st);
+    if (conv) launch_tile<64, 64, 1, 1, true, true>(c, part, p.S, p.kchunk, st);
+    else launch_tile<64, 64, 1, 1, false, true>(c, part, p.S, p.kchunk, st);
     const int64_t MN = (int64_t)c.M * c.N;
     const int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
     linear_f32_split_reduce<<<blocks, 256, 0, st>>>(c.out, c.ldo, part, p.S, c.M, c.N, c.bias, c.act, c.accumulate,
