@@ -423,10 +423,12 @@ void launch_dp_actions(float* out, const float* x, int start, int chunk, int A, 
 // out [Hout*Wout, Cout] = the k x k conv of the NHWC map x with W [Cout][k*k*Cin]
 // (im2col's column order) as one implicit GEMM; false when the shape or
 // alignment does not suit it (the caller then runs im2col + launch_linear_f32,
-// which gives the same values)
+// which gives the same values). resid [Hout*Wout, Cout] (not out): the output
+// is max(0, v + resid), bit for bit launch_add_relu's
 bool launch_conv_f32_implicit(float* out, const float* x, int H, int Wd, int Cin, int k, int stride, int pad,
                               int Hout, int Wout, const float* W, const float* bias, int Cout, int act,
-                              hipStream_t st, float* work = nullptr, size_t work_floats = 0);
+                              hipStream_t st, float* work = nullptr, size_t work_floats = 0,
+                              const float* resid = nullptr);
 // floats of npix im2col rows of K columns (rows padded to 4 floats), rounded up
 // to 64 floats so what follows stays 256-byte aligned
 inline size_t col_rows_floats(size_t npix, int K) { return (npix * (size_t)((K + 3) & ~3) + 63) / 64 * 64; }

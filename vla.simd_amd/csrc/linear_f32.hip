@@ -113,6 +113,8 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // one tap, and its tap advances by the slab's channels. Same
 // products in the same order as im2col + this kernel; no column matrix.
 // VEC: rows are 16-byte aligned runs; otherwise elements are loaded one by one.
+// resid (a block's skip map, rows as out's): out = relu(v + resid), the pass
+// that would read both again.
 // G = 2: two groups of four waves take half of the block's K slabs each, with
 // slabs, scales and sums of their own; the sums meet in LDS and each group
 // finishes half of the tile. Twice the waves where the tiles alone leave a CU
@@ -127,7 +129,8 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
                                                         const float* __restrict__ W, int ldw,
                                                         const float* __restrict__ bias, int M, int N,
                                                         int K, int act, int accumulate, float alpha,
-                                                        ConvGeom cg, float* __restrict__ part, int kchunk) {
+                                                        ConvGeom cg, const float* __restrict__ resid,
+                                                        float* __restrict__ part, int kchunk) {
     constexpr int BK = 32 * KS, LR = 8 * KS, ROWS = BM + BN;  // LR lanes hold a row of a slab
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
     constexpr int AV = BM * BK / 4 / 256, BV = BN * BK / 4 / 256;  // float4 loads per thread
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
     auto& sm = smem[grp];
     auto& unit = units[grp];
     auto& guess = guesses[grp];
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     // split K (part != null): chunk blockIdx.z of kchunk columns, raw sums into
@@ -404,6 +407,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
             }
             float* o = dst + (size_t)m * ldd + n;
             if (!part) v = act_of(v + (bias ? bias[n] : 0.0f), act);
+            if (resid && !part) v = relu_gt(v + resid[(size_t)m * ldd + n]);
             *o = !part && accumulate ? fmaf(alpha, v, *o) : v;
         }
         return;
@@ -440,6 +444,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
 
     // lane: row m = r16 of a fragment, columns n = 4 g .. 4 g + 3
     const bool vec = (ldd & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
+    const bool rvec = (ldd & 3) == 0 && (reinterpret_cast<uintptr_t>(resid) & 15) == 0;
 #pragma unroll
     for (int j = 0; j < FN; j++) {
         const int n = n0 + wn * TN + j * 16 + 4 * g;
@@ -459,6 +464,19 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
             for (int r = 0; r < 4; r++) {
                 v[r] = G > 1 ? acc[i][j][r] : acc[i][j][r] * (ua * unit[BM + wn * TN + j * 16 + 4 * g + r]);
                 if (!part) v[r] = act_of(v[r] + b[r], act);
+            }
+            if (resid && !part) {
+                const float* q = resid + (size_t)m * ldd + n;
+                if (rvec && n + 4 <= N) {
+                    const float4 d = *reinterpret_cast<const float4*>(q);
+                    v[0] = relu_gt(v[0] + d.x);
+                    v[1] = relu_gt(v[1] + d.y);
+                    v[2] = relu_gt(v[2] + d.z);
+                    v[3] = relu_gt(v[3] + d.w);
+                } else {
+                    for (int r = 0; r < 4; r++)
+                        if (n + r < N) v[r] = relu_gt(v[r] + q[r]);
+                }
             }
             if (vec && n + 4 <= N) {
                 if (!part && accumulate) {
@@ -620,13 +638,15 @@ void launch_skinny(float* out, int ldo, const float* x, int ldx, const float* W,
 __global__ __launch_bounds__(256) void linear_f32_split_reduce(float* __restrict__ out, int ldo,
                                                                const float* __restrict__ part, int S, int M, int N,
                                                                const float* __restrict__ bias, int act,
-                                                               int accumulate, float alpha) {
+                                                               int accumulate, float alpha,
+                                                               const float* __restrict__ resid) {
     const int64_t MN = (int64_t)M * N;
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < MN; e += (int64_t)gridDim.x * blockDim.x) {
         float v = part[e];
         for (int z = 1; z < S; z++) v += part[z * MN + e];
         const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
         v = act_of(v + (bias ? bias[n] : 0.0f), act);
+        if (resid) v = relu_gt(v + resid[(size_t)m * ldo + n]);
         float* o = out + (size_t)m * ldo + n;
         *o = accumulate ? fmaf(alpha, v, *o) : v;
     }
@@ -645,6 +665,7 @@ struct F32Call {
     int M, N, K, act, accumulate;
     float alpha;
     ConvGeom cg;
+    const float* resid = nullptr;
 };
 
 // Split-K plan for M > 128 over K >= 1024 when 64 x 64 tiles number < 128
@@ -671,7 +692,8 @@ template <int BM, int BN, int KS, int G, bool CONV, bool VEC>
 void launch_tile(const F32Call& c, float* part, int S, int kchunk, hipStream_t st) {
     const dim3 grid((c.N + BN - 1) / BN, (c.M + BM - 1) / BM, S);
     linear_f32_tiled<BM, BN, KS, G, CONV, VEC><<<grid, 256 * G, 0, st>>>(c.out, c.ldo, c.x, c.ldx, c.W, c.ldw, c.bias, c.M, c.N,
-                                                              c.K, c.act, c.accumulate, c.alpha, c.cg, part, kchunk);
+                                                              c.K, c.act, c.accumulate, c.alpha, c.cg, c.resid,
+                                                                     part, kchunk);
     VLA_LAUNCH_CHECK();
 }
 
@@ -706,7 +728,7 @@ void launch_f32_split(const F32Call& c, bool conv, const F32Split& p, float* par
     const int64_t MN = (int64_t)c.M * c.N;
     const int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
     linear_f32_split_reduce<<<blocks, 256, 0, st>>>(c.out, c.ldo, part, p.S, c.M, c.N, c.bias, c.act, c.accumulate,
-                                                    c.alpha);
+                                                    c.alpha, c.resid);
     VLA_LAUNCH_CHECK();
 }
 
@@ -762,7 +784,7 @@ void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float
 
 bool launch_conv_f32_implicit(float* out, const float* x, int H, int Wd, int Cin, int k, int stride, int pad,
                               int Hout, int Wout, const float* W, const float* bias, int Cout, int act,
-                              hipStream_t st, float* work, size_t work_floats) {
+                              hipStream_t st, float* work, size_t work_floats, const float* resid) {
     const char* e = std::getenv("VLA_CONV_F32_IMPLICIT");  // 0: im2col + GEMM (A/B runs)
     if (e && e[0] == '0' && e[1] == '\0') return false;
     VLA_REQUIRE(out && x && W && H > 0 && Wd > 0 && Cin > 0 && k > 0 && stride > 0 && pad >= 0 && Cout > 0 &&
@@ -779,7 +801,7 @@ bool launch_conv_f32_implicit(float* out, const float* x, int H, int Wd, int Cin
     if (M <= 128) return false;
     const ConvGeom cg{H, Wd, Cin, k, stride, pad, Wout};
     const F32Split sp = f32_split_plan(M, N, K);
-    const F32Call c{out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg};
+    const F32Call c{out, N, x, K, W, K, bias, M, N, K, act, 0, 1.0f, cg, resid};
     if (sp.S > 1) {  // as launch_linear_f32: split over K with a workspace, else not here
         if (!(work && work_floats >= (size_t)sp.S * M * N && aligned(work, 16))) return false;
         launch_f32_split(c, true, sp, work, st);

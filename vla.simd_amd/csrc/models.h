@@ -149,9 +149,10 @@ private:
     // maxima of |x| its producer wrote, out_part receives those of the relu'd
     // output; returns their count (0 when none are written). The ReLU runs
     // in the conv's epilogue where its kernel fuses it, else as a pass. resid
-    // (an int8 conv without ReLU or GroupNorm): the block's residual, added
+    // (a conv without ReLU or GroupNorm): the block's residual, added
     // and ReLU'd in the epilogue where the kernel fuses that (*resid_done =
-    // true, the maxima then those of the sum); otherwise the caller adds it.
+    // true, an int8 conv's maxima then those of the sum); otherwise the caller
+    // adds it.
     // ConvArgs of an int8 conv over x [H, W, cin] into out, with the trunk's workspace
     ConvArgs i8_args(const Conv& c, const float* x, int H, int W, float* out, const float* in_part,
                      int in_nparts) const;
