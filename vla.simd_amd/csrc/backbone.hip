@@ -98,9 +98,12 @@ __global__ __launch_bounds__(256) void im2col_f32x4_kernel(float* __restrict__ c
 }
 
 // The same columns for any Cin (the 3-channel stem) with K <= 256 and 32-bit
-// sizes: a wave per output pixel, its lanes walking the row (coalesced
-// stores), each lane's taps (ky, kx, ci) decomposed once; values identical
-// to im2col_f32_kernel's.
+// sizes: a wave per four output pixels at a time, its lanes walking the rows
+// (coalesced stores), each lane's taps (ky, kx, ci) decomposed once; values
+// identical to im2col_f32_kernel's. Bound by the loads' latency and by those
+// divisions: with one pixel per wave 76800 x 147 took 31.6 us, with four in
+// flight and the waves of kIm2colBlocks blocks walking on 17.8.
+constexpr int kIm2colBlocks = 2048;
 __global__ __launch_bounds__(256) void im2col_f32_rows_kernel(float* __restrict__ col, int ldc,
                                                               const float* __restrict__ x, int H, int Wd, int Cin,
                                                               int k, int stride, int pad, int Wout, int npix) {
@@ -114,17 +117,31 @@ __global__ __launch_bounds__(256) void im2col_f32_rows_kernel(float* __restrict_
         dy[j] = t / k;
         dx[j] = t - dy[j] * k;
     }
-    for (int p = blockIdx.x * 4 + (threadIdx.x >> 6); p < npix; p += gridDim.x * 4) {
-        const int oy = p / Wout, ox = p - oy * Wout;
-        const int y0 = oy * stride - pad, x0 = ox * stride - pad;
-        float* crow = col + (size_t)p * ldc;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int p = 4 * (blockIdx.x * 4 + wave); p < npix; p += gridDim.x * 16) {
+        int oy = p / Wout, ox = p - oy * Wout;
+        float v[4][4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = lane + 64 * j;
-            if (r >= K) break;
-            const int iy = y0 + dy[j], ix = x0 + dx[j];
-            const bool in = iy >= 0 && iy < H && ix >= 0 && ix < Wd;
-            crow[r] = in ? x[(iy * Wd + ix) * Cin + ci[j]] : 0.0f;
+        for (int i = 0; i < 4; i++) {  // (pixels past the last: loads masked by the row, nothing stored)
+            const int y0 = oy * stride - pad, x0 = ox * stride - pad;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int iy = y0 + dy[j], ix = x0 + dx[j];
+                const bool in = lane + 64 * j < K && iy >= 0 && iy < H && ix >= 0 && ix < Wd;
+                v[i][j] = in ? x[(iy * Wd + ix) * Cin + ci[j]] : 0.0f;
+            }
+            if (++ox == Wout) {
+                ox = 0;
+                ++oy;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (p + i >= npix) break;
+            float* crow = col + (size_t)(p + i) * ldc;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (lane + 64 * j < K) crow[lane + 64 * j] = v[i][j];
         }
     }
 }
@@ -332,7 +349,7 @@ void launch_im2col_f32(float* col, int ldc, const float* x, int H, int Wd, int C
                                                           (int)t4);
     } else if (K <= 256 && (int64_t)H * Wd * Cin < INT32_MAX && (int64_t)Hout * Wout < INT32_MAX) {
         const int npix = Hout * Wout;
-        const int blocks = (npix + 3) / 4 < 16384 ? (npix + 3) / 4 : 16384;
+        const int blocks = (npix + 15) / 16 < kIm2colBlocks ? (npix + 15) / 16 : kIm2colBlocks;
         im2col_f32_rows_kernel<<<blocks, 256, 0, st>>>(col, ldc, x, H, Wd, Cin, k, stride, pad, Wout, npix);
     } else {
         im2col_f32_kernel<<<grid_for(total), 256, 0, st>>>(col, ldc, x, H, Wd, Cin, k, stride, pad, Wout, total);
