@@ -101,8 +101,10 @@ __global__ __launch_bounds__(256) void im2col_f32x4_kernel(float* __restrict__ c
 // sizes: a wave per four output pixels at a time, its lanes walking the rows
 // (coalesced stores), each lane's taps (ky, kx, ci) decomposed once; values
 // identical to im2col_f32_kernel's. Bound by the loads' latency and by those
-// divisions: with one pixel per wave 76800 x 147 took 31.6 us, with four in
-// flight and the waves of kIm2colBlocks blocks walking on 17.8.
+// divisions: 76800 x 147 took 31.6 us with a wave per pixel, 17.8 with four
+// pixels' loads in flight and at most kIm2colBlocks blocks (eight per CU), whose
+// waves walk on with their taps. What is left is 45 MB of stores (9 us at the
+// copy rate) and as many 4-byte loads.
 constexpr int kIm2colBlocks = 2048;
 __global__ __launch_bounds__(256) void im2col_f32_rows_kernel(float* __restrict__ col, int ldc,
                                                               const float* __restrict__ x, int H, int Wd, int Cin,

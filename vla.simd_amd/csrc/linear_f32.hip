@@ -1,4 +1,4 @@
-// linear_f32.hip - fp32 linear layers on the fp32 matrix cores (gfx950).
+// linear_f32.hip - fp32 linear layers on the matrix cores (gfx950).
 //
 // out[m, n] (+)= act(sum_k x[m, k] * W[n, k] + bias[n])
 //
