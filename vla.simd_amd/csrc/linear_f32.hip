@@ -18,6 +18,7 @@
 
 #include "act.h"
 #include "common.h"
+#include "convgeom.h"
 #include "wave.h"
 
 #include <cstdlib>
@@ -119,10 +120,6 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // slabs, scales and sums of their own; the sums meet in LDS and each group
 // finishes half of the tile. Twice the waves where the tiles alone leave a CU
 // one block (4800 x 1152 x 128 21.6 -> 18.3 us).
-struct ConvGeom {
-    int H, Wd, Cin, k, stride, pad, Wout;
-};
-
 template <int BM, int BN, int KS, int G, bool CONV, bool VEC>
 __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ out, int ldo,
                                                         const float* __restrict__ x, int ldx,
@@ -297,10 +294,8 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
         first_tap();
 #pragma unroll
         for (int j = 0; j < AV; j++) {
-            const int iy = iy0[j] + cg.pad, ix = ix0[j] + cg.pad;
-            const bool in = iy < cg.H && ix < cg.Wd;  // (not with a kernel reaching past the far border only)
-            ma[j] = absmax4(0.0f, in ? *reinterpret_cast<const float4*>(x + ((size_t)iy * cg.Wd + ix) * cg.Cin + kq)
-                                     : make_float4(0.f, 0.f, 0.f, 0.f));
+            const int o = guess_offset(cg, iy0[j] + cg.pad, ix0[j] + cg.pad, kq);
+            ma[j] = absmax4(0.0f, o >= 0 ? *reinterpret_cast<const float4*>(x + o) : make_float4(0.f, 0.f, 0.f, 0.f));
         }
     }
     gload(0);
