@@ -94,7 +94,8 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // (2-norm, N(0, 1) rows, K = 768: 3.6e-7 against 5.8e-7).
 //
 // Every row of x and of W has a scale of its own, a power of two taken out of
-// the sums exactly. It is guessed from the row's values in one slab (the first;
+// the sums exactly (both at once and by the exponent: the product of the two
+// need not be a float). It is guessed from the row's values in one slab (the first;
 // a convolution's centre tap, which always lies inside the image), so that they
 // reach 2^12, or from the tile's where the row has none; the maxima of all
 // slabs are kept, and a tile some row of which ends up outside [2^8, 2^15] is
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
     constexpr int AV = BM * BK / 4 / 256, BV = BN * BK / 4 / 256;  // float4 loads per thread
     static_assert(AV >= 1 && BV >= 1 && TM % 16 == 0 && TN % 16 == 0 && FM % G == 0, "tile");
     __shared__ __attribute__((aligned(16))) char smem[G][2][2][KS][ROWS * 64];
-    __shared__ float units[G][ROWS];  // what a row's sums are multiplied by in the end
+    __shared__ int units[G][ROWS];  // the power of two a row's sums are multiplied by in the end
     __shared__ uint32_t guesses[G][2];  // the tile's largest value of x and of W in the guess slab
     const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     auto& sm = smem[grp];
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
             const float t = mx * exp_float(e);
             off = off || !(mx == 0.0f || (t >= 256.0f && t <= 32768.0f));
             inf = inf || !(mx <= 3.4028235e38f);
-            if (tid % LR == 0) unit[r] = exp_float(254u - e);
+            if (tid % LR == 0) unit[r] = 127 - (int)e;
         };
 #pragma unroll
         for (int j = 0; j < AV; j++) check(ma[j], ea[j], (tid + 256 * j) / LR);
@@ -419,9 +420,9 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
 #pragma unroll
             for (int j = 0; j < FN; j++) {
                 v4f v = grp ? acc[i][j] : acc[FG + i][j];  // the other group's half
-                const float ua = unit[wm * TM + (grp ? i : FG + i) * 16 + r16];
+                const int ua = unit[wm * TM + (grp ? i : FG + i) * 16 + r16];
 #pragma unroll
-                for (int r = 0; r < 4; r++) v[r] *= ua * unit[BM + wn * TN + j * 16 + 4 * g + r];
+                for (int r = 0; r < 4; r++) v[r] = ldexpf(v[r], ua + unit[BM + wn * TN + j * 16 + 4 * g + r]);
                 mine[(i * FN + j) * 256] = v;
             }
         __syncthreads();
@@ -430,9 +431,9 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
 #pragma unroll
             for (int j = 0; j < FN; j++) {
                 v4f v = grp ? acc[FG + i][j] : acc[i][j];
-                const float ua = unit[wm * TM + (grp ? FG + i : i) * 16 + r16];
+                const int ua = unit[wm * TM + (grp ? FG + i : i) * 16 + r16];
 #pragma unroll
-                for (int r = 0; r < 4; r++) v[r] *= ua * unit[BM + wn * TN + j * 16 + 4 * g + r];
+                for (int r = 0; r < 4; r++) v[r] = ldexpf(v[r], ua + unit[BM + wn * TN + j * 16 + 4 * g + r]);
                 acc[i][j] = v + other[(i * FN + j) * 256];
             }
     }
@@ -453,11 +454,11 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
             const int fr = wm * TM + (grp * FG + i) * 16 + r16, m = m0 + fr;
             if (m >= M) continue;
             float* o = dst + (size_t)m * ldd + n;
-            const float ua = unit[fr];
+            const int ua = unit[fr];
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                v[r] = G > 1 ? acc[i][j][r] : acc[i][j][r] * (ua * unit[BM + wn * TN + j * 16 + 4 * g + r]);
+                v[r] = G > 1 ? acc[i][j][r] : ldexpf(acc[i][j][r], ua + unit[BM + wn * TN + j * 16 + 4 * g + r]);
                 if (!part) v[r] = act_of(v[r] + b[r], act);
             }
             if (resid && !part) {
