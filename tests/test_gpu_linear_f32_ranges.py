@@ -39,3 +39,18 @@ def test_whole_numbers_times_powers(vla, M, K, N, ex, ew):
     W = np.ldexp(r.integers(-15, 16, (N, K)), ew).astype(np.float32)
     want = x.astype(np.float64) @ W.astype(np.float64).T
     assert np.array_equal(vla.dense_linear(x, W, None), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_outlier_columns(vla, M, K, N):
+    """A few channels 4 to 1000 times the others, outside the first 64 columns: the
+    sums keep the rows' precision whichever pass finds them."""
+    r = np.random.default_rng(3)
+    x, W = r.standard_normal((M, K), dtype=np.float32), r.standard_normal((N, K), dtype=np.float32)
+    for c, f in ((70, 4), (75, 30), (90, 1000)):
+        x[:, c] *= np.float32(f)
+    W[::5, 80] *= np.float32(300)
+    got = vla.dense_linear(x, W, None)
+    want = x.astype(np.float64) @ W.astype(np.float64).T
+    size = np.linalg.norm(x.astype(np.float64), axis=1)[:, None] * np.linalg.norm(W.astype(np.float64), axis=1)[None]
+    assert float((np.abs(got - want) / size).max()) < 2e-6

@@ -97,10 +97,10 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // the sums exactly (both at once and by the exponent: the product of the two
 // need not be a float). It is guessed from the row's values in one slab (the first;
 // a convolution's centre tap, which always lies inside the image), so that they
-// reach 2^12, or from the tile's where the row has none; the maxima of all
-// slabs are kept, and a tile some row of which ends up outside [2^8, 2^15] is
+// reach 2^6, or from the tile's where the row has none; the maxima of all
+// slabs are kept, and a tile some row of which ends up outside [2^3, 2^15] is
 // computed once more with the scales of the true maxima. So no part overflows
-// and no operand loses more than 2^-33 of its row's largest value (2^-22 of
+// and no operand loses more than 2^-28 of its row's largest value (2^-22 of
 // itself at worst). Infinities are left to plain fmaf chains.
 //
 // BM x BN tiles, four waves in a 2 x 2 grid. A K slab, KS steps of 32, is loaded as
@@ -328,9 +328,9 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
         for (int j = 0; j < BV; j++) mb[j] = mb[j] > 0.0f ? mb[j] : __uint_as_float(guess[1]);
     }
 #pragma unroll
-    for (int j = 0; j < AV; j++) ea[j] = scale_exp(ma[j], 12);
+    for (int j = 0; j < AV; j++) ea[j] = scale_exp(ma[j], 6);
 #pragma unroll
-    for (int j = 0; j < BV; j++) eb[j] = scale_exp(mb[j], 12);
+    for (int j = 0; j < BV; j++) eb[j] = scale_exp(mb[j], 6);
 
     bool again = false, bad;
     for (;;) {
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
         auto check = [&](float& mx, uint32_t e, int r) {
             mx = lanes_max<LR>(mx);
             const float t = mx * exp_float(e);
-            off = off || !(mx == 0.0f || (t >= 256.0f && t <= 32768.0f));
+            off = off || !(mx == 0.0f || (t >= 8.0f && t <= 32768.0f));
             inf = inf || !(mx <= 3.4028235e38f);
             if (tid % LR == 0) unit[r] = 127 - (int)e;
         };
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
 #pragma unroll
         for (int j = 0; j < BV; j++) check(mb[j], eb[j], BM + (tid + 256 * j) / LR);
         // a second pass can only find values that are not finite, or rows so
-        // small that 2^126 leaves them below 2^8
+        // small that 2^126 leaves them below 2^3
         bad = __syncthreads_or(again ? inf : off);
         if (!bad || again) break;
         again = true;
