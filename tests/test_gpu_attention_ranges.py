@@ -1,0 +1,109 @@
+"""Masked attention where its numbers leave the ordinary range: additive masks of
+large finite values, scores past the point where floats are whole numbers apart,
+queries and keys of zeros or nearly so, blocked keys that hold anything.
+
+Against double-precision softmax. A mask value m leaves a score s + m its fp32
+rounding, half an ulp of m: where that matters the expectation is taken from the
+rounded scores. Tolerance: fp32 sums, 2e-6 of the result's 2-norm (2e-7 is seen).
+"""
+
+import math
+
+import numpy as np
+import pytest
+
+from test_gpu_attention import LOWEST, naive
+
+pytestmark = pytest.mark.gpu
+
+HD = 64
+
+
+def rel(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+def qkv(seed, sq, sk, nq=2, nkv=2, hd=HD):
+    r = np.random.default_rng(seed)
+    return tuple(r.standard_normal((n, h * hd), dtype=np.float32) for n, h in ((sq, nq), (sk, nkv), (sk, nkv)))
+
+
+def rounded(Q, K, V, nq, nkv, hd, scale, mask):
+    """naive() with the scores rounded to fp32 where the mask is added."""
+    sq, sk = len(Q), len(K)
+    q, k, v = (x.astype(np.float64).reshape(len(x), -1, hd) for x in (Q, K, V))
+    out = np.zeros((sq, nq, hd))
+    for h in range(nq):
+        s = (q[:, h] @ k[:, h // (nq // nkv)].T * scale).astype(np.float32)
+        with np.errstate(over="ignore"):
+            s = np.where(mask == LOWEST, np.float32(-np.inf), s + mask).astype(np.float64)
+        mx = s.max(axis=1, keepdims=True)
+        with np.errstate(invalid="ignore"):
+            e = np.where(np.isneginf(s), 0.0, np.exp(s - mx))
+        z = e.sum(axis=1, keepdims=True)
+        out[:, h] = np.where(z == 0, v[:, h // (nq // nkv)].mean(axis=0), (e @ v[:, h // (nq // nkv)]) / np.where(z == 0, 1, z))
+    return out.reshape(sq, nq * hd)
+
+
+@pytest.mark.parametrize("sq,sk", [(1, 33), (20, 70), (50, 300), (700, 300)])
+@pytest.mark.parametrize("m", [-1e4, -3e6, -1e7, -3e7, -1e8, -1e9, -1e30])
+def test_large_finite_masks(vla, m, sq, sk):
+    """Padding written as an additive value: trailing and leading key ranges (whole
+    32-key tiles of a wave among them), single keys, and rows with nothing else."""
+    Q, K, V = qkv(sq + sk, sq, sk)
+    r = np.random.default_rng(2)
+    mask = np.zeros((sq, sk), np.float32)
+    mask[0::4, sk // 3:] = m
+    mask[1::4, :sk // 2 + 3] = m
+    mask[2::4][r.random((len(mask[2::4]), sk)) < 0.3] = m
+    mask[3::8] = m
+    mask[7::8] = m
+    mask[7::8, sk // 2] = LOWEST
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125, kind=vla.MASK_DENSE, dense=mask)
+    want = rounded(Q, K, V, 2, 2, HD, 0.125, mask)
+    mine = np.abs(got - want).max(axis=1)
+    # where every key carries the mask the weights hang on the last bit of s + m,
+    # whose product and sum may round once or twice: one step either way
+    whole = (mask != 0).all(axis=1)
+    assert np.isfinite(got).all()
+    assert rel(got[~whole], want[~whole]) < 2e-6, mine.max()
+    ulp = float(np.spacing(np.float32(-m)))
+    if whole.any():
+        if ulp > 64:  # every score is absorbed: the weights are equal
+            assert rel(got[whole], want[whole]) < 2e-6
+        else:
+            bound = 2 * np.expm1(min(2.0, ulp)) * np.abs(V).max() + 1e-5
+            assert mine[whole].max() < bound
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "groups", "dense"])
+@pytest.mark.parametrize("size", [1e7, 1e8, 1e10, 1e20])
+def test_scores_past_whole_numbers(vla, size, kind):
+    """Scores whose floats lie more than one apart: the largest takes all."""
+    sq, sk = 40, 300
+    Q, K, V = qkv(9, sq, sk)
+    Q = (Q * np.float32(size)).astype(np.float32)
+    kw, keep = {}, np.ones((sq, sk), bool)
+    if kind == "causal":
+        keep = np.arange(sk)[None] <= np.arange(sq)[:, None] + 5
+        kw = dict(kind=vla.MASK_CAUSAL, causal_offset=5)
+    elif kind == "groups":
+        r = np.random.default_rng(1)
+        qg, kg = r.integers(0, 9, sq).astype(np.uint8), r.integers(0, 9, sk).astype(np.uint8)
+        allow = (r.random((9, 9)) < 0.5).astype(np.uint8)
+        allow[np.arange(9), np.arange(9)] = 1
+        keep = allow[qg][:, kg].astype(bool)
+        kw = dict(kind=vla.MASK_GROUPS, q_group=qg, k_group=kg, allow=allow.reshape(-1))
+    elif kind == "dense":
+        kw = dict(kind=vla.MASK_DENSE, dense=np.zeros((sq, sk), np.float32))
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125, **kw)
+    assert np.isfinite(got).all()
+    want = naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))
+    # rows whose two largest scores lie apart by more than the scores' fp32 error
+    q, k = (x.astype(np.float64).reshape(-1, 2, HD) for x in (Q, K))
+    for h in range(2):
+        s = np.where(keep, q[:, h] @ k[:, h].T * 0.125, -np.inf)
+        top = np.sort(s, axis=1)[:, -2:]
+        clear = top[:, 1] - top[:, 0] > 40 + 4e-6 * np.linalg.norm(q[:, h], axis=1) * np.linalg.norm(k[:, h], axis=1).max() * 0.125
+        assert clear.sum() > sq // 2
+        assert rel(got[clear, h * HD:(h + 1) * HD], want[clear, h * HD:(h + 1) * HD]) < 2e-6

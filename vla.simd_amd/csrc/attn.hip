@@ -1062,9 +1062,10 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             vlim = 32768.0f * uv;
         }
 
-        // scale, mask and online softmax in the log2 domain: t = acc f + mask
-        // log2 e, p = 2^(t - M) with one rounding in the exponent; the rounding
-        // of M is common to a query's weights and leaves with the division
+        // scale, mask and online softmax in the log2 domain: x = acc f + mask
+        // log2 e, rounded once; the maximum and the weights p = 2^(x - M) are
+        // taken from the same x, so no weight passes 1 (a mask of -1e9 leaves
+        // x and M whole multiples of 64, the unrounded score is not)
         Split8 pp[QF];
         const bool plain = MKC == 0 && mk == 0 && qfull && kv0 + 32 <= kv_end;  // wave-uniform
 #pragma unroll
@@ -1081,8 +1082,9 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                         const float v = mval[f][kt][r];
                         const bool blocked =
                             qi >= a.seq_q || kv0 + 16 * kt + 4 * g + r >= kv_end || v == -FLT_MAX;
-                        mval[f][kt][r] = blocked ? -INFINITY : v * kLog2e;
-                        mt = fmaxf(mt, fmaf(sacc[f][kt][r], fq, mval[f][kt][r]));
+                        const float x = blocked ? -INFINITY : fmaf(sacc[f][kt][r], fq, v * kLog2e);
+                        sacc[f][kt][r] = x;
+                        mt = fmaxf(mt, x);
                     }
             } else {
                 if (!plain) {
@@ -1097,7 +1099,9 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                             sacc[f][kt][r] = blocked ? -INFINITY : sacc[f][kt][r];
                         }
                 }
-                mt = max4(sacc[f][0], sacc[f][1]) * fq;
+                sacc[f][0] *= fq;
+                sacc[f][1] *= fq;
+                mt = max4(sacc[f][0], sacc[f][1]);
             }
             const float mnew = fmaxf(M[f], rows_max(mt));
             // a query that has seen nothing yet keeps M = -inf; its weights are
@@ -1109,7 +1113,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             for (int kt = 0; kt < 2; kt++) {
                 auto weight = [&](int r) {
                     // times 2^15 after the exponential: 15 in the exponent would coarsen it
-                    return fast_exp2(fmaf(sacc[f][kt][r], fq, MKC == 1 ? mval[f][kt][r] - mref : -mref)) * 32768.0f;
+                    return fast_exp2(sacc[f][kt][r] - mref) * 32768.0f;
                 };
                 x[kt] = make_float4(weight(0), weight(1), weight(2), weight(3));
             }
