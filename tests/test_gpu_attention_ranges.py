@@ -107,3 +107,41 @@ def test_scores_past_whole_numbers(vla, size, kind):
         clear = top[:, 1] - top[:, 0] > 40 + 4e-6 * np.linalg.norm(q[:, h], axis=1) * np.linalg.norm(k[:, h], axis=1).max() * 0.125
         assert clear.sum() > sq // 2
         assert rel(got[clear, h * HD:(h + 1) * HD], want[clear, h * HD:(h + 1) * HD]) < 2e-6
+
+
+def masks_of(vla, kind, sq, sk):
+    if kind == "causal":
+        return dict(kind=vla.MASK_CAUSAL, causal_offset=2), np.arange(sk)[None] <= np.arange(sq)[:, None] + 2
+    if kind == "groups":
+        qg, kg = (np.arange(sq) % 5).astype(np.uint8), (np.arange(sk) // 7 % 5).astype(np.uint8)
+        allow = np.tril(np.ones((5, 5), np.uint8))
+        return dict(kind=vla.MASK_GROUPS, q_group=qg, k_group=kg, allow=allow.reshape(-1)), allow[qg][:, kg].astype(bool)
+    if kind == "dense":
+        keep = np.random.default_rng(5).random((sq, sk)) < 0.6
+        return dict(kind=vla.MASK_DENSE, dense=np.where(keep, 0, LOWEST).astype(np.float32)), keep
+    return {}, np.ones((sq, sk), bool)
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "groups", "dense"])
+@pytest.mark.parametrize("q,k", [(0, 0), (0, 1), (1, 0), (0, 2.0 ** -9), (1e-20, 1e-20), (1e-30, 1e-15), (1e-38, 1e-38)])
+@pytest.mark.parametrize("sq,sk", [(5, 33), (40, 300)])
+def test_zero_and_tiny_scores(vla, kind, q, k, sq, sk):
+    """Queries and keys of zeros or whose products underflow: equal weights."""
+    Q, K, V = qkv(11, sq, sk)
+    Q, K = (Q * np.float32(q)).astype(np.float32), (K * np.float32(k)).astype(np.float32)
+    kw, keep = masks_of(vla, kind, sq, sk)
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125, **kw)
+    assert rel(got, naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))) < 2e-6
+
+
+@pytest.mark.parametrize("kind", ["causal", "groups", "dense"])
+def test_some_zero_rows(vla, kind):
+    """Zero query rows and zero 32-key tiles among ordinary ones."""
+    sq, sk = 70, 300
+    Q, K, V = qkv(12, sq, sk)
+    Q[3::5] = 0
+    K[64:128] = 0
+    K *= np.float32(2.0 ** -10)
+    kw, keep = masks_of(vla, kind, sq, sk)
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125, **kw)
+    assert rel(got, naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))) < 2e-6

@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
 #pragma unroll
         for (int f = 0; f < QF; f++) {
             const int qi = q0 + 16 * f + c;
-            const float fq = fs[f] * uk;  // > 0
+            const float fq = fs[f] * uk;
             float mt;
             if constexpr (MKC == 1) {
                 mt = -INFINITY;
@@ -1087,7 +1087,9 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                         mt = fmaxf(mt, x);
                     }
             } else {
-                if (!plain) {
+                sacc[f][0] *= fq;
+                sacc[f][1] *= fq;
+                if (!plain) {  // (after the product: fq underflows to 0 under zero or tiny operands)
 #pragma unroll
                     for (int kt = 0; kt < 2; kt++)
 #pragma unroll
@@ -1099,8 +1101,6 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                             sacc[f][kt][r] = blocked ? -INFINITY : sacc[f][kt][r];
                         }
                 }
-                sacc[f][0] *= fq;
-                sacc[f][1] *= fq;
                 mt = max4(sacc[f][0], sacc[f][1]);
             }
             const float mnew = fmaxf(M[f], rows_max(mt));
