@@ -76,6 +76,21 @@ def test_large_finite_masks(vla, m, sq, sk):
             assert mine[whole].max() < bound
 
 
+@pytest.mark.parametrize("low", [-2.4e38, -3.3e38, -3.3895314e38])
+def test_masks_next_to_lowest(vla, low):
+    """Values between lowest() and its quotient by log2 e are additive like any
+    other (bf16's lowest is one): only lowest() and -inf block."""
+    sq, sk = 40, 200
+    Q, K, V = qkv(3, sq, sk)
+    low = np.float32(low)
+    mask = np.full((sq, sk), LOWEST, np.float32)
+    mask[:, 20:90] = low
+    mask[::2, 150] = 0
+    mask[1::4, 40:60] = low * np.float32(0.9)
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125, kind=vla.MASK_DENSE, dense=mask)
+    assert rel(got, rounded(Q, K, V, 2, 2, HD, 0.125, mask)) < 2e-6
+
+
 @pytest.mark.parametrize("kind", ["none", "causal", "groups", "dense"])
 @pytest.mark.parametrize("size", [1e7, 1e8, 1e10, 1e20])
 def test_scores_past_whole_numbers(vla, size, kind):

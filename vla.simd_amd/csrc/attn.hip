@@ -790,7 +790,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
 
     // the query fragments: query 16 f + c, dims 32 s + 8 g ..
     Split8 qreg[C::QLDS ? 1 : QF][C::QLDS ? 1 : S];
-    float fs[QF];  // scores' unit of a query, times the softmax scale and log2 e
+    float fs[QF];  // scores' unit of a query, times the softmax scale
     f16x8* qlds = reinterpret_cast<f16x8*>(smem);
     float* fsl = reinterpret_cast<float*>(reinterpret_cast<char*>(smem) + C::FSB);
     auto qload = [&](int f, float4 (&x)[S][2]) {
@@ -807,7 +807,6 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
     };
     bool bad = false;
     // splits a query fragment; returns its scores' unit times the softmax scale
-    // and log2 e
     auto qsplit = [&](const float4 (&x)[S][2], Split8 (&q)[S]) {
         float mx = 0.0f;
 #pragma unroll
@@ -819,7 +818,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
         const uint32_t e = scale_exp(mx);
 #pragma unroll
         for (int s = 0; s < S; s++) q[s] = split8(x[s][0], x[s][1], a.scale < 0.0f ? -exp_float(e) : exp_float(e));
-        return exp_float(254u - e) * fabsf(a.scale) * kLog2e;
+        return exp_float(254u - e) * fabsf(a.scale);
     };
     // the queries' loads ahead of the first tile's: loads return in order
     const bool qmine = !C::QLDS || wave < QF;
@@ -881,7 +880,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
 #pragma unroll
         for (int f = 0; f < QF; f++) fs[f] = fsl[16 * f + c];
 
-    float M[QF], lsum[QF];  // running max (times log2 e) and sum per query 16 f + c
+    float M[QF], lsum[QF];  // running max and sum per query 16 f + c
     v4f oacc[QF][U][4];     // O^T: dim 64 u + 4 (4 g + r) + dt of query 16 f + c,
                             // in units of 1 / sv (both sums carry the weights' 2^15)
     // K's and V's scales: the first tile's, until a value outgrows them (V's
@@ -1062,10 +1061,12 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             vlim = 32768.0f * uv;
         }
 
-        // scale, mask and online softmax in the log2 domain: x = acc f + mask
-        // log2 e, rounded once; the maximum and the weights p = 2^(x - M) are
-        // taken from the same x, so no weight passes 1 (a mask of -1e9 leaves
-        // x and M whole multiples of 64, the unrounded score is not)
+        // scale, mask and online softmax: x = acc f + mask in the natural domain
+        // (times log2 e a mask between lowest() / log2 e and lowest(), bf16's
+        // lowest among them, would overflow), rounded once; the maximum and the
+        // weights p = e^(x - M) are taken from the same x, so no weight passes 1
+        // (a mask of -1e9 leaves x and M whole multiples of 64, the unrounded
+        // score is not)
         Split8 pp[QF];
         const bool plain = MKC == 0 && mk == 0 && qfull && kv0 + 32 <= kv_end;  // wave-uniform
 #pragma unroll
@@ -1082,7 +1083,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                         const float v = mval[f][kt][r];
                         const bool blocked =
                             qi >= a.seq_q || kv0 + 16 * kt + 4 * g + r >= kv_end || v == -FLT_MAX;
-                        const float x = blocked ? -INFINITY : fmaf(sacc[f][kt][r], fq, v * kLog2e);
+                        const float x = blocked ? -INFINITY : fmaf(sacc[f][kt][r], fq, v);
                         sacc[f][kt][r] = x;
                         mt = fmaxf(mt, x);
                     }
@@ -1105,15 +1106,15 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             }
             const float mnew = fmaxf(M[f], rows_max(mt));
             // a query that has seen nothing yet keeps M = -inf; its weights are
-            // 2^-inf = 0 against any finite reference
+            // e^-inf = 0 against any finite reference
             const float mref = fmaxf(mnew, -FLT_MAX);
-            const float decay = fast_exp2(M[f] - mref), alpha = decay * resc;
+            const float decay = fast_exp2((M[f] - mref) * kLog2e), alpha = decay * resc;
             float4 x[2];
 #pragma unroll
             for (int kt = 0; kt < 2; kt++) {
                 auto weight = [&](int r) {
                     // times 2^15 after the exponential: 15 in the exponent would coarsen it
-                    return fast_exp2(sacc[f][kt][r] - mref) * 32768.0f;
+                    return fast_exp2((sacc[f][kt][r] - mref) * kLog2e) * 32768.0f;
                 };
                 x[kt] = make_float4(weight(0), weight(1), weight(2), weight(3));
             }
@@ -1165,7 +1166,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
 #pragma unroll
     for (int f = 0; f < QF; f++) lsum[f] = rows_sum(lsum[f]);
 
-    // merge the waves' partial states: M*, then sum_w 2^(M_w - M*) (l_w, O_w)
+    // merge the waves' partial states: M*, then sum_w e^(M_w - M*) (l_w, O_w)
     __syncthreads();
     float* Mm = smem;                   // [W][NQ]
     float* Ml = smem + W * NQ;          // [W][NQ]
@@ -1210,7 +1211,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
         float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < W; w++) {
-            const float fw = mw[w] == -INFINITY ? 0.0f : fast_exp2(mw[w] - ms);
+            const float fw = mw[w] == -INFINITY ? 0.0f : fast_exp2((mw[w] - ms) * kLog2e);
             l += fw * Ml[w * NQ + q];
             const float4 v = *reinterpret_cast<const float4*>(Mo + (w * NQ + q) * MO + 4 * d4);
             o.x += fw * v.x;
