@@ -160,3 +160,36 @@ def test_some_zero_rows(vla, kind):
     kw, keep = masks_of(vla, kind, sq, sk)
     got = vla.attention(Q, K, V, 2, 2, HD, 0.125, **kw)
     assert rel(got, naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))) < 2e-6
+
+
+@pytest.mark.parametrize("what", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("kind", ["causal", "groups", "dense", "dense-inf"])
+def test_not_finite_behind_a_mask(vla, kind, what):
+    """Infinities and NaN in a key or value reach only the queries that see it."""
+    sq, sk = 140, 300
+    Q, K, V = qkv(14, sq, sk)
+    at = 100
+    if kind == "causal":
+        keep = np.arange(sk)[None] <= np.arange(sq)[:, None]
+        kw = dict(kind=vla.MASK_CAUSAL, causal_offset=0)
+    else:
+        qg = (np.arange(sq) >= 60).astype(np.uint8)
+        keep = np.ones((sq, sk), bool)
+        keep[:60, at - 5:at + 9] = False
+        if kind == "groups":
+            kg = np.zeros(sk, np.uint8)
+            kg[at - 5:at + 9] = 1
+            kw = dict(kind=vla.MASK_GROUPS, q_group=qg, k_group=kg, allow=np.array([1, 0, 1, 1], np.uint8))
+        else:
+            kw = dict(kind=vla.MASK_DENSE, dense=np.where(keep, 0, LOWEST if kind == "dense" else -np.inf).astype(np.float32))
+    want = naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))
+    blind = ~keep[:, at]
+    assert blind.sum() >= 60
+    for x in (K, V):
+        y = x.copy()
+        y[at, 3] = what
+        got = vla.attention(Q, y if x is K else K, y if x is V else V, 2, 2, HD, 0.125, **kw)
+        assert rel(got[blind], want[blind]) < 2e-6
+        assert rel(got[:, HD:], want[:, HD:]) < 2e-6  # the other head
+        if x is V:
+            assert rel(got[:, 4:], want[:, 4:]) < 2e-6 and not np.isfinite(got[~blind, 3]).any()

@@ -546,8 +546,8 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 // The loads of a wave's next tile are issued as soon as the registers of this
 // one are split.
 //
-// Infinities (and NaN) in an operand: such a block is computed again from the
-// inputs in plain fp32 (attn_block_f32).
+// Infinities in an operand, and outputs that are not finite: such a block is
+// computed again from the inputs in plain fp32 (attn_block_f32).
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -622,7 +622,7 @@ __device__ __forceinline__ bool mask_blocks(const AttnArgs& a, int qi, int j, fl
     if (a.mask_kind == 1) {
         const float mv = a.mask[(size_t)qi * a.ldm + j];
         *add = mv;
-        return mv == -FLT_MAX;
+        return mv <= -FLT_MAX;  // lowest() or -inf
     }
     if (a.mask_kind == 2) return j > qi + a.causal_offset;
     if (a.mask_kind == 3) return !a.allow[(int)a.q_group[qi] * a.n_groups + a.k_group[j]];
@@ -631,7 +631,8 @@ __device__ __forceinline__ bool mask_blocks(const AttnArgs& a, int qi, int j, fl
 
 // The block's queries [q0, q0 + nq) of head h in plain fp32, one query per wave
 // at a time, lanes over keys, then over dims: for operands the split kernel
-// does not carry, whose speed does not matter.
+// does not carry, whose speed does not matter. Keys a query may not see are
+// left out, whatever they hold.
 template <int HDP>
 __device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq, int h, int kvh) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -659,11 +660,12 @@ __device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq
         for (int u = 0; u < HDP / 64; u++) o[u] = 0.0f;
         for (int j0 = 0; j0 < a.seq_k; j0 += 64) {
             const int j = j0 + lane;
-            float p = 0.0f;
-            if (j < a.seq_k) p = masked ? 1.0f : fast_exp2((score(j) - m) * kLog2e);
+            float p = 0.0f, add;
+            const bool seen = j < a.seq_k && (masked || !mask_blocks(a, qi, j, &add));
+            if (seen) p = masked ? 1.0f : fast_exp2((score(j) - m) * kLog2e);
             l += p;
-            const int n = a.seq_k - j0 < 64 ? a.seq_k - j0 : 64;
-            for (int t = 0; t < n; t++) {
+            for (uint64_t left = __ballot(seen); left; left &= left - 1) {
+                const int t = __ffsll((unsigned long long)left) - 1;
                 const float pt = __shfl(p, t);
 #pragma unroll
                 for (int u = 0; u < HDP / 64; u++) {
@@ -1082,7 +1084,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                     for (int r = 0; r < 4; r++) {
                         const float v = mval[f][kt][r];
                         const bool blocked =
-                            qi >= a.seq_q || kv0 + 16 * kt + 4 * g + r >= kv_end || v == -FLT_MAX;
+                            qi >= a.seq_q || kv0 + 16 * kt + 4 * g + r >= kv_end || v <= -FLT_MAX;
                         const float x = blocked ? -INFINITY : fmaf(sacc[f][kt][r], fq, v);
                         sacc[f][kt][r] = x;
                         mt = fmaxf(mt, x);
@@ -1186,17 +1188,19 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
                                 oacc[f][u][3][r] * uv);
     }
     __syncthreads();
-    if (*flags) {  // block-uniform
-        attn_block_f32<HDP>(a, q0, NQ, h, kvh);
-        return;
-    }
-    // thread x writes float4 column x % (HDP / 4) of queries x / (HDP / 4), ...:
+    // thread x finishes float4 column x % (HDP / 4) of queries x / (HDP / 4), ...:
     // whole 16-byte runs of an output row per wave
     constexpr int QPT = W * 64 / (HDP / 4);  // queries per step of the block
-    const int d4 = tid % (HDP / 4);
-    bool any_masked = false;
-    for (int q = tid / (HDP / 4); q < NQ; q += QPT) {
-        if (q0 + q >= a.seq_q) break;
+    constexpr int NO = (NQ + QPT - 1) / QPT;
+    const int d4 = tid % (HDP / 4), part = tid / (HDP / 4);
+    float4 o[NO];
+    uint32_t masked = 0;  // bit n: no key of query part + n QPT counts
+    bool odd = *flags != 0;
+#pragma unroll
+    for (int n = 0; n < NO; n++) {
+        const int q = part + n * QPT;
+        o[n] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (q >= NQ || q0 + q >= a.seq_q) continue;
         float mw[W], ms = -INFINITY;
 #pragma unroll
         for (int w = 0; w < W; w++) {
@@ -1204,46 +1208,37 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             ms = fmaxf(ms, mw[w]);
         }
         if (ms == -INFINITY) {
-            any_masked = true;
+            masked |= 1u << n;
             continue;
         }
         float l = 0.0f;
-        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < W; w++) {
             const float fw = mw[w] == -INFINITY ? 0.0f : fast_exp2((mw[w] - ms) * kLog2e);
             l += fw * Ml[w * NQ + q];
             const float4 v = *reinterpret_cast<const float4*>(Mo + (w * NQ + q) * MO + 4 * d4);
-            o.x += fw * v.x;
-            o.y += fw * v.y;
-            o.z += fw * v.z;
-            o.w += fw * v.w;
+            o[n].x += fw * v.x;
+            o[n].y += fw * v.y;
+            o[n].z += fw * v.z;
+            o[n].w += fw * v.w;
         }
         const float inv = 1.0f / l;
-        if (4 * d4 < HD)
-            *reinterpret_cast<float4*>(a.out + (size_t)(q0 + q) * a.ldo + h * HD + 4 * d4) =
-                make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+        o[n] = make_float4(o[n].x * inv, o[n].y * inv, o[n].z * inv, o[n].w * inv);
+        odd = odd || !(fabsf(o[n].x) + fabsf(o[n].y) + fabsf(o[n].z) + fabsf(o[n].w) < INFINITY);
     }
-    // rows with every key blocked: the uniform mean of V over all seq_k keys,
-    // the same for each of them, from partial sums over 4 W strided key sets
-    if (__syncthreads_or(any_masked)) {
-        // the partial sums take Mm's place: each thread first notes which of its
-        // queries are masked
-        uint32_t mine = 0;
-        int n = 0;
-        for (int q = tid / (HDP / 4); q < NQ; q += QPT, n++) {
-            if (q0 + q >= a.seq_q) break;
-            float ms = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < W; w++) ms = fmaxf(ms, Mm[w * NQ + q]);
-            if (ms == -INFINITY) mine |= 1u << n;
+    if (__syncthreads_or(odd || masked)) {
+        // not finite: from an input that this query sees, or 0 times one that
+        // it does not
+        if (__syncthreads_or(odd)) {
+            attn_block_f32<HDP>(a, q0, NQ, h, kvh);
+            return;
         }
-        __syncthreads();
-        constexpr int NP = W * 64 / (HDP / 4);
-        const int part = tid / (HDP / 4);
+        // rows with every key blocked: the uniform mean of V over all seq_k keys,
+        // the same for each of them, from partial sums over 4 W strided key sets
+        // (in Mm's place: every thread is past it)
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
         if (4 * d4 < HD)
-            for (int j = part; j < a.seq_k; j += NP) {
+            for (int j = part; j < a.seq_k; j += QPT) {
                 const float4 v = *reinterpret_cast<const float4*>(Vb + (size_t)j * a.ldv + 4 * d4);
                 sum.x += v.x;
                 sum.y += v.y;
@@ -1253,7 +1248,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
         *reinterpret_cast<float4*>(smem + part * HDP + 4 * d4) = sum;
         __syncthreads();
         float4 mean = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int x = 0; x < NP; x++) {
+        for (int x = 0; x < QPT; x++) {
             const float4 v = *reinterpret_cast<const float4*>(smem + x * HDP + 4 * d4);
             mean.x += v.x;
             mean.y += v.y;
@@ -1261,11 +1256,15 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             mean.w += v.w;
         }
         const float inv = 1.0f / (float)a.seq_k;
-        n = 0;
-        for (int q = part; q < NQ; q += QPT, n++)
-            if (((mine >> n) & 1u) && 4 * d4 < HD)
-                *reinterpret_cast<float4*>(a.out + (size_t)(q0 + q) * a.ldo + h * HD + 4 * d4) =
-                    make_float4(mean.x * inv, mean.y * inv, mean.z * inv, mean.w * inv);
+#pragma unroll
+        for (int n = 0; n < NO; n++)
+            if ((masked >> n) & 1u) o[n] = make_float4(mean.x * inv, mean.y * inv, mean.z * inv, mean.w * inv);
+    }
+#pragma unroll
+    for (int n = 0; n < NO; n++) {
+        const int q = part + n * QPT;
+        if (q < NQ && q0 + q < a.seq_q && 4 * d4 < HD)
+            *reinterpret_cast<float4*>(a.out + (size_t)(q0 + q) * a.ldo + h * HD + 4 * d4) = o[n];
     }
 }
 
