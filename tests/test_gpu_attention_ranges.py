@@ -162,6 +162,37 @@ def test_some_zero_rows(vla, kind):
     assert rel(got, naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, np.where(keep, 0, -np.inf).astype(np.float32))) < 2e-6
 
 
+@pytest.mark.parametrize("kind", ["causal", "groups", "dense"])
+@pytest.mark.parametrize("which", ["k", "v", "kv"])
+@pytest.mark.parametrize("size", [1e3, 1e5, 1e6, 1e12, 1e30, 3e38])
+def test_blocked_keys_of_any_size(vla, kind, which, size):
+    """Rows that the mask blocks for every query (padding, the stale end of a cache)
+    may hold any finite value: they weigh exactly nothing, and the others keep
+    their full precision."""
+    sq, sk = 40, 200
+    Q, K, V = qkv(13, sq, sk)
+    if kind == "causal":
+        keep = np.arange(sk)[None] <= np.arange(sq)[:, None] + 20
+        kw = dict(kind=vla.MASK_CAUSAL, causal_offset=20)
+    else:
+        pad = np.zeros(sk, bool)
+        pad[[0, 1, 17, 40, 95]] = True
+        pad[130:150] = True
+        keep = np.broadcast_to(~pad, (sq, sk))
+        if kind == "groups":
+            kw = dict(kind=vla.MASK_GROUPS, q_group=np.zeros(sq, np.uint8), k_group=pad.astype(np.uint8),
+                      allow=np.array([1, 0, 0, 0], np.uint8))
+        else:
+            kw = dict(kind=vla.MASK_DENSE, dense=np.where(keep, 0, LOWEST).astype(np.float32))
+    out = ~keep.any(axis=0)
+    mask = np.where(keep, 0, -np.inf).astype(np.float32)
+    want = naive(Q, K, V, sq, sk, 2, 2, HD, 0.125, mask)
+    for x, name in ((K, "k"), (V, "v")):
+        if name in which:
+            x[out] = np.sign(x[out]) * np.float32(size)
+    assert rel(vla.attention(Q, K, V, 2, 2, HD, 0.125, **kw), want) < 2e-6
+
+
 @pytest.mark.parametrize("what", [np.inf, -np.inf, np.nan])
 @pytest.mark.parametrize("kind", ["causal", "groups", "dense", "dense-inf"])
 def test_not_finite_behind_a_mask(vla, kind, what):
@@ -193,3 +224,29 @@ def test_not_finite_behind_a_mask(vla, kind, what):
         assert rel(got[:, HD:], want[:, HD:]) < 2e-6  # the other head
         if x is V:
             assert rel(got[:, 4:], want[:, 4:]) < 2e-6 and not np.isfinite(got[~blind, 3]).any()
+
+
+@pytest.mark.parametrize("what", ["q", "k"])
+@pytest.mark.parametrize("size", [1e-36, 1e36])
+def test_scores_of_far_operands(vla, what, size):
+    """Queries and keys near opposite ends of the range, their scores ordinary."""
+    sq, sk = 40, 200
+    Q, K, V = qkv(16, sq, sk)
+    f = np.float32(size)
+    Q, K = (Q * f, K / f) if what == "q" else (Q / f, K * f)
+    got = vla.attention(Q, K, V, 2, 2, HD, 0.125)
+    assert rel(got, naive(Q, K, V, sq, sk, 2, 2, HD, 0.125)) < 2e-6
+
+
+def test_operands_of_mixed_sizes(vla):
+    """Keys, values and their columns over 2^-30 .. 2^30 in one tile: each key's score
+    and each column's sum keep fp32's precision of their own size."""
+    sq, sk = 40, 300
+    Q, K, V = qkv(17, sq, sk)
+    r = np.random.default_rng(3)
+    cols = np.exp2(r.integers(-30, 31, V.shape[1])).astype(np.float32)
+    dims = np.exp2(r.integers(-30, 31, K.shape[1])).astype(np.float32)
+    got = vla.attention(Q / dims, K * dims, V * cols, 2, 2, HD, 0.125)
+    want = naive(Q / dims, K * dims, V * cols, sq, sk, 2, 2, HD, 0.125)
+    err = np.linalg.norm(got - want, axis=0) / np.linalg.norm(want, axis=0)
+    assert err.max() < 4e-6, err.max()

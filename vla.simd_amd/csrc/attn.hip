@@ -546,8 +546,9 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 // The loads of a wave's next tile are issued as soon as the registers of this
 // one are split.
 //
-// Infinities in an operand, and outputs that are not finite: such a block is
-// computed again from the inputs in plain fp32 (attn_block_f32).
+// Infinities in an operand, outputs that are not finite and operands whose values
+// lie too far apart for one scale: such a block is computed again from the inputs
+// in plain fp32 (attn_block_f32).
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -645,9 +646,14 @@ __device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq
             float add;
             if (mask_blocks(a, qi, j, &add)) return -INFINITY;
             const float* kp = a.K + (size_t)j * a.ldk + kvh * HD;
-            float s = 0.0f;
-            for (int d = 0; d < HD; d++) s = fmaf(qp[d], kp[d], s);
-            s *= a.scale;
+            float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+            for (int d = 0; d < HD; d += 4) {
+                const float4 k = *reinterpret_cast<const float4*>(kp + d);
+                s4 = make_float4(fmaf(qp[d], k.x, s4.x), fmaf(qp[d + 1], k.y, s4.y), fmaf(qp[d + 2], k.z, s4.z),
+                                 fmaf(qp[d + 3], k.w, s4.w));
+            }
+            const float s = ((s4.x + s4.y) + (s4.z + s4.w)) * a.scale;
             return a.mask_kind == 1 ? s + add : s;
         };
         float m = -INFINITY;
@@ -655,22 +661,34 @@ __device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq
         for (int o = 32; o; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
         const bool masked = m == -INFINITY;
         float l = 0.0f;
-        float o[HDP / 64];
+        float o[4][HDP / 64];  // four sums of every fourth key
 #pragma unroll
-        for (int u = 0; u < HDP / 64; u++) o[u] = 0.0f;
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int u = 0; u < HDP / 64; u++) o[t][u] = 0.0f;
         for (int j0 = 0; j0 < a.seq_k; j0 += 64) {
             const int j = j0 + lane;
             float p = 0.0f, add;
             const bool seen = j < a.seq_k && (masked || !mask_blocks(a, qi, j, &add));
             if (seen) p = masked ? 1.0f : fast_exp2((score(j) - m) * kLog2e);
             l += p;
-            for (uint64_t left = __ballot(seen); left; left &= left - 1) {
-                const int t = __ffsll((unsigned long long)left) - 1;
-                const float pt = __shfl(p, t);
+            // eight keys' loads in flight (past the last key: the last again, weight 0)
+            const uint64_t take = __ballot(seen);
+            for (int t0 = 0; t0 < 64 && j0 + t0 < a.seq_k; t0 += 8) {
+                float v[8][HDP / 64];
 #pragma unroll
-                for (int u = 0; u < HDP / 64; u++) {
-                    const int d = u * 64 + lane;
-                    if (d < HD) o[u] = fmaf(pt, a.V[(size_t)(j0 + t) * a.ldv + kvh * HD + d], o[u]);
+                for (int t = 0; t < 8; t++)
+#pragma unroll
+                    for (int u = 0; u < HDP / 64; u++) {
+                        const int d = u * 64 + lane;
+                        v[t][u] = d < HD ? a.V[(size_t)min(j0 + t0 + t, a.seq_k - 1) * a.ldv + kvh * HD + d] : 0.0f;
+                    }
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    const float pt = __shfl(p, t0 + t);
+#pragma unroll
+                    for (int u = 0; u < HDP / 64; u++)
+                        o[t & 3][u] = (take >> (t0 + t)) & 1u ? fmaf(pt, v[t][u], o[t & 3][u]) : o[t & 3][u];
                 }
             }
         }
@@ -678,7 +696,7 @@ __device__ __forceinline__ void attn_block_f32(const AttnArgs& a, int q0, int nq
 #pragma unroll
         for (int u = 0; u < HDP / 64; u++) {
             const int d = u * 64 + lane;
-            if (d < HD) a.out[(size_t)qi * a.ldo + h * HD + d] = o[u] / l;
+            if (d < HD) a.out[(size_t)qi * a.ldo + h * HD + d] = ((o[0][u] + o[1][u]) + (o[2][u] + o[3][u])) / l;
         }
     }
 }
@@ -999,6 +1017,10 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             sk = exp_float(e);
             uk = exp_float(254u - e);
             klim = 32768.0f * uk;
+            // queries and keys, seen or not, whose largest product could add 2^14 to
+            // a score: 2^-40 of that is no longer below the rounding of an ordinary one
+#pragma unroll
+            for (int f = 0; f < QF; f++) bad = bad || fs[f] * kmax > 1.0f;
         }
 
         // K's parts to the operand's lanes through this wave's LDS rows
@@ -1056,6 +1078,16 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
         if (__any(vmax > vlim)) {
             vmax = wave_max_f32(vmax);
             bad = bad || not_finite(vmax);
+            // a key's four columns (that are not zero, hence the bits less one) 2^17
+            // below the largest of a tile, as beside a row of padding that holds
+            // anything: a scale for both leaves those too few bits
+#pragma unroll
+            for (int jj = 0; jj < 8; jj++)
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const float m = absmax(absmax(0.0f, vr[jj][u].x, vr[jj][u].y), vr[jj][u].z, vr[jj][u].w);
+                    bad = bad || __float_as_uint(m) - 1u < __float_as_uint(vmax * 0x1p-17f);
+                }
             const uint32_t e = scale_exp(vmax);
             sv = exp_float(e);
             resc = uv * sv;  // the old unit over the new one (0 before any tile, whose sums are 0)
