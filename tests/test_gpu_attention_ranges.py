@@ -226,6 +226,23 @@ def test_not_finite_behind_a_mask(vla, kind, what):
             assert rel(got[:, 4:], want[:, 4:]) < 2e-6 and not np.isfinite(got[~blind, 3]).any()
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("size", [1e-36, 1e-33, 1e33, 1e36])
+def test_values_near_the_range_ends(vla, hd, size):
+    sq, sk = 40, 200
+    Q, K, V = qkv(15, sq, sk, hd=hd)
+    V = (V * np.float32(size)).astype(np.float32)
+    got = vla.attention(Q, K, V, 2, 2, hd, 1 / math.sqrt(hd))
+    want = naive(Q, K, V, sq, sk, 2, 2, hd, 1 / math.sqrt(hd))
+    assert rel(got / size, want / size) < 2e-6
+    one = V.copy()
+    one[:, 5] /= np.float32(size)  # a column of its own size keeps its own precision
+    got = vla.attention(Q, K, one, 2, 2, hd, 1 / math.sqrt(hd))
+    want = naive(Q, K, one, sq, sk, 2, 2, hd, 1 / math.sqrt(hd))
+    for cols, unit in ((np.arange(2 * hd) == 5, 1.0), (np.arange(2 * hd) != 5, size)):
+        assert rel(got[:, cols] / unit, want[:, cols] / unit) < 2e-6
+
+
 @pytest.mark.parametrize("what", ["q", "k"])
 @pytest.mark.parametrize("size", [1e-36, 1e36])
 def test_scores_of_far_operands(vla, what, size):

@@ -1069,12 +1069,25 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             VLA_QK(h, h)
 #undef VLA_QK
         }
+        // the largest of the lane's columns, and the least that is not zero (as
+        // bits less one)
         float vmax = 0.0f, resc = 1.0f;
+        uint32_t vmin = ~0u;
 #pragma unroll
-        for (int jj = 0; jj < 8; jj++)
+        for (int u = 0; u < U; u++) {
+            float m[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int u = 0; u < U; u++)
-                vmax = absmax(absmax(vmax, vr[jj][u].x, vr[jj][u].y), vr[jj][u].z, vr[jj][u].w);
+            for (int jj = 0; jj < 8; jj += 2) {
+                const float4 &p = vr[jj][u], &q = vr[jj + 1][u];
+                m[0] = absmax(m[0], p.x, q.x);
+                m[1] = absmax(m[1], p.y, q.y);
+                m[2] = absmax(m[2], p.z, q.z);
+                m[3] = absmax(m[3], p.w, q.w);
+            }
+            vmax = absmax(absmax(vmax, m[0], m[1]), m[2], m[3]);
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) vmin = min(vmin, __float_as_uint(m[dt]) - 1u);
+        }
         if (__any(vmax > vlim)) {
             vmax = wave_max_f32(vmax);
             bad = bad || not_finite(vmax);
@@ -1094,6 +1107,7 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             uv = exp_float(254u - e);
             vlim = 32768.0f * uv;
         }
+        bad = bad || vmin < __float_as_uint(0.125f * uv);  // a column of eight keys 2^18 below the scale
 
         // scale, mask and online softmax: x = acc f + mask in the natural domain
         // (times log2 e a mask between lowest() / log2 e and lowest(), bf16's
@@ -1205,19 +1219,22 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
     float* Mm = smem;                   // [W][NQ]
     float* Ml = smem + W * NQ;          // [W][NQ]
     float* Mo = smem + 2 * W * NQ;      // [W][NQ][MO]
+    // V's unit and the weights' 2^15 out of the sums, by the exponent: their
+    // quotient need not be a float
+    const int ve = (int)(__float_as_uint(uv) >> 23) - 127 - 15;
 #pragma unroll
     for (int f = 0; f < QF; f++) {
         if (g == 0) {
             Mm[wave * NQ + 16 * f + c] = M[f];
-            Ml[wave * NQ + 16 * f + c] = lsum[f];
+            Ml[wave * NQ + 16 * f + c] = lsum[f] * 0x1p-15f;
         }
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
                 *reinterpret_cast<float4*>(Mo + (wave * NQ + 16 * f + c) * MO + 64 * u + 16 * g + 4 * r) =
-                    make_float4(oacc[f][u][0][r] * uv, oacc[f][u][1][r] * uv, oacc[f][u][2][r] * uv,
-                                oacc[f][u][3][r] * uv);
+                    make_float4(ldexpf(oacc[f][u][0][r], ve), ldexpf(oacc[f][u][1][r], ve),
+                                ldexpf(oacc[f][u][2][r], ve), ldexpf(oacc[f][u][3][r], ve));
     }
     __syncthreads();
     // thread x finishes float4 column x % (HDP / 4) of queries x / (HDP / 4), ...:
