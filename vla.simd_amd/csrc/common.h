@@ -9,6 +9,8 @@
 #include <stdexcept>
 #include <string>
 
+#include "convgeom.h"
+
 namespace vla {
 namespace hip {
 
@@ -436,9 +438,12 @@ inline size_t col_rows_floats(size_t npix, int K) { return (npix * (size_t)((K +
 // use for this shape when one is passed; 0 when the shape is not split
 size_t linear_f32_split_floats(int M, int N, int K);
 // taps: x rows may overlap (ldx < K) as launch_quantize_rows' taps view
+// cols: x is im2col's rows of this convolution (they then give the implicit
+// form's values bit for bit)
 void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float* W, int ldw,
                        const float* bias, int M, int N, int K, int act, int accumulate, float alpha,
-                       hipStream_t st, float* work = nullptr, size_t work_floats = 0, bool taps = false);
+                       hipStream_t st, float* work = nullptr, size_t work_floats = 0, bool taps = false,
+                       const ConvGeom* cols = nullptr);
 
 // runtime.cpp
 hipStream_t library_stream();  // stream of the host-pointer forms

@@ -20,7 +20,7 @@ struct ConvGeom {
 // guess of a row's scale, kq (a multiple of 4) channels in; -1: nowhere. A slab
 // may be wider than a pixel (64 channels on maps of 32).
 VLA_HOST_DEVICE inline int guess_offset(const ConvGeom& cg, int iy, int ix, int kq) {
-    return kq < cg.Cin && iy < cg.H && ix < cg.Wd ? (iy * cg.Wd + ix) * cg.Cin + kq : -1;
+    return kq < cg.Cin && iy >= 0 && iy < cg.H && ix >= 0 && ix < cg.Wd ? (iy * cg.Wd + ix) * cg.Cin + kq : -1;
 }
 
 }  // namespace hip

@@ -112,7 +112,7 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // CONV: x is an NHWC map and row m of A is output pixel m's k x k patch,
 // column (ky * k + kx) * Cin + ci (im2col's order), gathered by the A loads
 // themselves: with Cin % 32 == 0 a thread's float4 of a slab always lies in
-// one tap, and its tap advances by the slab's channels. Same
+// one tap, and its tap advances by the slab's channels. Same scales and
 // products in the same order as im2col + this kernel; no column matrix.
 // VEC: rows are 16-byte aligned runs; otherwise elements are loaded one by one.
 // resid (a block's skip map, rows as out's): out = relu(v + resid), the pass
@@ -127,7 +127,8 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
                                                         const float* __restrict__ W, int ldw,
                                                         const float* __restrict__ bias, int M, int N,
                                                         int K, int act, int accumulate, float alpha,
-                                                        ConvGeom cg, const float* __restrict__ resid,
+                                                        ConvGeom cg, int gcol, int gn,
+                                                        const float* __restrict__ resid,
                                                         float* __restrict__ part, int kchunk) {
     constexpr int BK = 32 * KS, LR = 8 * KS, ROWS = BM + BN;  // LR lanes hold a row of a slab
     constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 16, FN = TN / 16;
@@ -289,19 +290,28 @@ __global__ __launch_bounds__(256 * G) void linear_f32_tiled(float* __restrict__ 
         }
     };
 
-    // the guess: rows' maxima in the first slab (CONV: x's from the centre tap)
+    // the guess: rows' maxima in the first slab, x's of a convolution from the
+    // centre tap: the map's pixel, or im2col's columns gcol .. gcol + gn - 1 (the
+    // same values, so both forms take the same scales)
     if (tid < 2) guess[tid] = 0;
-    if (CONV) {
-        first_tap();
+    const bool tap = CONV || (VEC && gn > 0);
+    if (CONV) first_tap();
+    if (tap) {
 #pragma unroll
         for (int j = 0; j < AV; j++) {
-            const int o = guess_offset(cg, iy0[j] + cg.pad, ix0[j] + cg.pad, kq);
-            ma[j] = absmax4(0.0f, o >= 0 ? *reinterpret_cast<const float4*>(x + o) : make_float4(0.f, 0.f, 0.f, 0.f));
+            const float* p = nullptr;
+            if (CONV) {
+                const int t = min(cg.pad, cg.k - 1), o = guess_offset(cg, iy0[j] + t, ix0[j] + t, kq);
+                if (o >= 0) p = x + o;
+            } else if (kq < gn) {
+                p = ap[j] - kbeg + gcol;
+            }
+            ma[j] = absmax4(0.0f, p ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f));
         }
     }
     gload(0);
 #pragma unroll
-    for (int j = 0; j < AV; j++) ma[j] = lanes_max<LR>(CONV ? ma[j] : absmax4(0.0f, ra[j]));
+    for (int j = 0; j < AV; j++) ma[j] = lanes_max<LR>(tap ? ma[j] : absmax4(0.0f, ra[j]));
 #pragma unroll
     for (int j = 0; j < BV; j++) mb[j] = lanes_max<LR>(absmax4(0.0f, rb[j]));
     bool none = false;  // a row without values in the guess slab takes the tile's guess
@@ -662,6 +672,7 @@ struct F32Call {
     float alpha;
     ConvGeom cg;
     const float* resid = nullptr;
+    int gcol = 0, gn = 0;  // the columns of x that a row's scale is guessed from (gn 0: the first slab's)
 };
 
 // Split-K plan for M > 128 over K >= 1024 when 64 x 64 tiles number < 128
@@ -688,8 +699,8 @@ template <int BM, int BN, int KS, int G, bool CONV, bool VEC>
 void launch_tile(const F32Call& c, float* part, int S, int kchunk, hipStream_t st) {
     const dim3 grid((c.N + BN - 1) / BN, (c.M + BM - 1) / BM, S);
     linear_f32_tiled<BM, BN, KS, G, CONV, VEC><<<grid, 256 * G, 0, st>>>(c.out, c.ldo, c.x, c.ldx, c.W, c.ldw, c.bias, c.M, c.N,
-                                                              c.K, c.act, c.accumulate, c.alpha, c.cg, c.resid,
-                                                                     part, kchunk);
+                                                              c.K, c.act, c.accumulate, c.alpha, c.cg, c.gcol, c.gn,
+                                                                     c.resid, part, kchunk);
     VLA_LAUNCH_CHECK();
 }
 
@@ -737,7 +748,7 @@ size_t linear_f32_split_floats(int M, int N, int K) {
 
 void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float* W, int ldw,
                        const float* bias, int M, int N, int K, int act, int accumulate, float alpha,
-                       hipStream_t st, float* work, size_t work_floats, bool taps) {
+                       hipStream_t st, float* work, size_t work_floats, bool taps, const ConvGeom* cols) {
     VLA_REQUIRE(M >= 0 && N > 0 && K > 0, "linear_f32: need M >= 0, N > 0, K > 0");
     VLA_REQUIRE((ldx >= K || (taps && ldx > 0)) && ldw >= K && ldo >= N,
                 "linear_f32: row strides shorter than the rows");
@@ -751,7 +762,13 @@ void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float
         VLA_LAUNCH_CHECK();
         return;
     }
-    const F32Call c{out, ldo, x, ldx, W, ldw, bias, M, N, K, act, accumulate, alpha, ConvGeom{}};
+    F32Call c{out, ldo, x, ldx, W, ldw, bias, M, N, K, act, accumulate, alpha, ConvGeom{}};
+    if (cols && cols->Cin % 32 == 0) {  // as the implicit form guesses (which takes no other widths)
+        const int t = cols->pad < cols->k ? cols->pad : cols->k - 1;
+        c.gcol = (t * cols->k + t) * cols->Cin;
+        c.gn = cols->Cin;
+        VLA_REQUIRE(c.gcol + c.gn <= K, "linear_f32: the columns are not these patches'");
+    }
     const bool vec = ldx % 4 == 0 && ldw % 4 == 0 && aligned(x, 16) && aligned(W, 16);
     if (!vec) {
         launch_tiles<false, false>(c, st);

@@ -328,8 +328,9 @@ void OctoStem::encode_dev(const uint8_t* img, float* out, hipStream_t st) {
                                           0, st, part, part_f)) {
                 const int ldc = kpad4(K);
                 launch_im2col_f32(col_, ldc, a_, L.H, L.W, L.cin, k_, stride_, pad_, L.Ho, L.Wo, st);
+                const ConvGeom cg{L.H, L.W, L.cin, k_, stride_, pad_, L.Wo};
                 launch_linear_f32(b_, L.cout, col_, ldc, L.W_, K, L.b, L.Ho * L.Wo, L.cout, K, 0, 0, 1.0f, st, part,
-                                  part_f);
+                                  part_f, false, &cg);
             }
         }
         launch_groupnorm(a_, b_, L.gs, L.gb, L.Ho * L.Wo, L.cout, groups_, gn_eps_, true, gA_, gB_, gW_, gw_doubles_,

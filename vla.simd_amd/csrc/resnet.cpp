@@ -326,8 +326,9 @@ int ResNetTrunk::conv(const Conv& c, const float* x, int H, int W, float* out, b
                 launch_im2col_f32(col_, ldx, x, H, W, c.cin, c.k, c.stride, c.pad, Ho, Wo, st);
                 rows = col_;
             }
+            const ConvGeom cg{H, W, c.cin, c.k, c.stride, c.pad, Wo};
             launch_linear_f32(out, c.cout, rows, ldx, c.W, c.ldw, c.b, Ho * Wo, c.cout, K, conv_relu ? 1 : 0, 0, 1.0f, st,
-                              part, part_f);
+                              part, part_f, false, plain ? nullptr : &cg);
         }
     }
     if (c.gs)
