@@ -66,6 +66,10 @@ def oracle():
     return _orc
 
 
+class ReferenceMissing(Exception):
+    """A comparison with the reference's own build was asked for and there is none."""
+
+
 def ref_available() -> bool:
     return os.path.exists(REF_PATH)
 
@@ -74,7 +78,7 @@ def ref():
     global _ref
     if _ref is None:
         if not ref_available():
-            raise RuntimeError(f"{REF_PATH} missing: run make -C oracle ref (needs the reference sources)")
+            raise ReferenceMissing(f"{REF_PATH} missing: run make -C oracle ref (needs the reference sources)")
         L = ctypes.CDLL(REF_PATH)
         P, i, f = c_void_p, c_int, c_float
         L.ref_int8_available.restype = i
