@@ -1107,7 +1107,10 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             uv = exp_float(254u - e);
             vlim = 32768.0f * uv;
         }
-        bad = bad || vmin < __float_as_uint(0.125f * uv);  // a column of eight keys 2^18 below the scale
+        // a column of the lane's keys 2^18 below the scale. (Not of fewer than four, the
+        // last ones, where the lane's others lie past them: of 64 ordinary values one
+        // is that small every few hundred calls, of four keys' none.)
+        bad = bad || (kv0 + 4 * g + 3 < a.seq_k && vmin < __float_as_uint(0.125f * uv));
 
         // scale, mask and online softmax: x = acc f + mask in the natural domain
         // (times log2 e a mask between lowest() / log2 e and lowest(), bf16's
