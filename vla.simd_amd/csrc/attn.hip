@@ -37,6 +37,7 @@
 // the reference forms them); exp(x) is evaluated as v_exp_f32(x * log2 e).
 
 #include "common.h"
+#include "fp16parts.h"
 #include "wave.h"
 
 #include <cfloat>
@@ -550,22 +551,10 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 // lie too far apart for one scale: such a block is computed again from the inputs
 // in plain fp32 (attn_block_f32).
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
 struct Split8 {
     f16x8 h, m;
 };
 
-// The two parts of x0 and x1, packed. (v_fma_mix{lo,hi}_f16 would scale, round
-// and subtract at once, but they issue at half rate: 8 cycles against 4 for
-// v_cvt_pk_f16_f32 and v_fma_mix_f32.)
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m) {
-    float r0, r1;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(x0), "v"(x1));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(h), "v"(x0));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(h), "v"(x1));
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(m) : "v"(r0), "v"(r1));
-}
 __device__ __forceinline__ Split8 split8(const float4& x, const float4& y) {
     uint4 h, m;
     split2(x.x, x.y, h.x, m.x);
@@ -578,12 +567,6 @@ __device__ __forceinline__ Split8 split8(const float4& x, const float4& y, float
     return split8(make_float4(x.x * s, x.y * s, x.z * s, x.w * s), make_float4(y.x * s, y.y * s, y.z * s, y.w * s));
 }
 
-// max(m, |x|, |y|); NaN is passed over
-__device__ __forceinline__ float absmax(float m, float x, float y) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x), "v"(y));
-    return m;
-}
-
 // max over eight values (NaN is passed over)
 __device__ __forceinline__ float max4(v4f x, v4f y) {
     float m;
@@ -593,15 +576,7 @@ __device__ __forceinline__ float max4(v4f x, v4f y) {
     return fmaxf(m, y[3]);
 }
 
-// Biased exponent of the power of two that brings values up to `mx` below 2^15
-// (fp16 ends at 65504); 254 minus it is its inverse's. Zero and the smallest
-// values take the largest that has an inverse.
-__device__ __forceinline__ uint32_t scale_exp(float mx) {
-    const uint32_t e = (__float_as_uint(mx) >> 23) & 0xffu;
-    return e < 15 ? 253u : 268u - e;
-}
 __device__ __forceinline__ bool not_finite(float mx) { return ((__float_as_uint(mx) >> 23) & 0xffu) == 255u; }
-__device__ __forceinline__ float exp_float(uint32_t e) { return __uint_as_float(e << 23); }
 
 // n / d for 0 <= n < 2^20, given the float nearest 1 / d: (n + 0.5) / d is at
 // least 0.5 / d away from the whole numbers, the rounding below n 2^-23 / d
@@ -832,10 +807,10 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
 #pragma unroll
         for (int s = 0; s < S; s++)
 #pragma unroll
-            for (int e = 0; e < 2; e++) mx = absmax(absmax(mx, x[s][e].x, x[s][e].y), x[s][e].z, x[s][e].w);
+            for (int e = 0; e < 2; e++) mx = absmax4(mx, x[s][e]);
         mx = rows_max(mx);
         bad = bad || not_finite(mx);
-        const uint32_t e = scale_exp(mx);
+        const uint32_t e = scale_exp(mx, 14);
 #pragma unroll
         for (int s = 0; s < S; s++) q[s] = split8(x[s][0], x[s][1], a.scale < 0.0f ? -exp_float(e) : exp_float(e));
         return exp_float(254u - e) * fabsf(a.scale);
@@ -1009,11 +984,11 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
         for (int jj = 0; jj < 8; jj++)
 #pragma unroll
             for (int u = 0; u < U; u++)
-                kmax = absmax(absmax(kmax, kr[jj][u].x, kr[jj][u].y), kr[jj][u].z, kr[jj][u].w);
+                kmax = absmax4(kmax, kr[jj][u]);
         if (__any(kmax > klim)) {
             kmax = wave_max_f32(kmax);
             bad = bad || not_finite(kmax);
-            const uint32_t e = scale_exp(kmax);
+            const uint32_t e = scale_exp(kmax, 14);
             sk = exp_float(e);
             uk = exp_float(254u - e);
             klim = 32768.0f * uk;
@@ -1098,10 +1073,10 @@ __global__ __launch_bounds__(W * 64, HDP == 64 ? 2 : 1) void attn_split(AttnArgs
             for (int jj = 0; jj < 8; jj++)
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const float m = absmax(absmax(0.0f, vr[jj][u].x, vr[jj][u].y), vr[jj][u].z, vr[jj][u].w);
+                    const float m = absmax4(0.0f, vr[jj][u]);
                     bad = bad || __float_as_uint(m) - 1u < __float_as_uint(vmax * 0x1p-17f);
                 }
-            const uint32_t e = scale_exp(vmax);
+            const uint32_t e = scale_exp(vmax, 14);
             sv = exp_float(e);
             resc = uv * sv;  // the old unit over the new one (0 before any tile, whose sums are 0)
             uv = exp_float(254u - e);

@@ -18,7 +18,7 @@
 
 #include "act.h"
 #include "common.h"
-#include "convgeom.h"
+#include "fp16parts.h"
 #include "wave.h"
 
 #include <cstdlib>
@@ -31,26 +31,6 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// The two fp16 parts of a float scaled by a power of two: x s = h + m + e, h =
-// fp16(x s), m = fp16(x s - h), |e| <= 2^-22 |x s| or 2^-25 (half of fp16's
-// smallest step), whichever is more.
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m) {
-    float r0, r1;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(x0), "v"(x1));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(h), "v"(x0));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(h), "v"(x1));
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(m) : "v"(r0), "v"(r1));
-}
-
-// max(m, |x|, |y|, |z|, |w|); NaN is passed over
-__device__ __forceinline__ float absmax4(float m, const float4& v) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.x), "v"(v.y));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.z), "v"(v.w));
-    return m;
-}
-
 // max over the N = 8 or 16 lanes that hold a row
 template <int N>
 __device__ __forceinline__ float lanes_max(float v) {
@@ -59,14 +39,6 @@ __device__ __forceinline__ float lanes_max(float v) {
     v = fmaxf(v, dpp_f32<0x141, 0xf>(v, v));   // row_half_mirror
     return N == 8 ? v : fmaxf(v, dpp_f32<0x140, 0xf>(v, v));  // row_mirror
 }
-
-// The power of two that brings `mx` to [2^top, 2^(top + 1)), as its biased
-// exponent, kept where it and its inverse (254 minus it) are normal floats.
-__device__ __forceinline__ uint32_t scale_exp(float mx, int top) {
-    const int e = 254 + top - (int)((__float_as_uint(mx) >> 23) & 0xffu);
-    return (uint32_t)(e < 1 ? 1 : e > 253 ? 253 : e);
-}
-__device__ __forceinline__ float exp_float(uint32_t e) { return __uint_as_float(e << 23); }
 
 // Block barrier that orders LDS only: __syncthreads' release fence would also
 // wait for the global loads of the slab after next.
