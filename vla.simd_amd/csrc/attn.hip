@@ -7,13 +7,14 @@
 //   score is -inf gets weight exactly 0;  out = sum_j softmax_j * v_j;  a row
 //   with every key blocked is the uniform mean of V over all seq_k keys
 //   (attn_uniform_row, avx2/attn.cpp:45-52).
-// fp32 throughout; results are tolerance-class against the reference (its exp
-// is a Cephes polynomial, its sums run in another order).
+// fp32 operands, sums and softmax; results are tolerance-class against the
+// reference (its exp is a Cephes polynomial, its sums run in another order).
 //
 // Two kernels: attn_split (below, head_dim <= 128) forms both products from
-// fp16 parts of the fp32 values, attn_fwd from the values themselves on the
-// fp32 matrix cores; it keeps head_dim 129 to 256 and the calls the split form
-// does not take (scale 0 or not finite, strides or lengths past its offsets).
+// two fp16 parts of the fp32 values, 22 bits of each, attn_fwd from the values
+// themselves on the fp32 matrix cores; it keeps head_dim 129 to 256 and the calls
+// the split form does not take (scales that are not finite, strides or lengths past
+// its offsets).
 //
 // attn_fwd: a block owns 16 queries of one head; its W waves split the key range: wave w
 // takes key tiles w, w + W, ... (KT keys each), stages each tile in its own
@@ -514,18 +515,27 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // attn_split: the same attention with both products on the fp16 matrix cores.
 //
-// Scaled by a power of two, a float x is h + m + e with h = fp16(x), m =
-// fp16(x - h) and |e| <= 2^-22 |x| (2^-24.5 in the mean, and no more than 2^-40
-// of the largest value that shares the scale, fp16's subnormals included). A
-// product of two floats is hh + hm + mh to that accuracy, so three
+// The operands' two parts (fp16parts.h) hold them to 2^-22 (2^-24.5 in the mean)
+// or to 2^-40 of the largest value that shares the scale, whichever is more. So three
 // v_mfma_f32_16x16x32_f16 (16 cycles each, exact products, fp32 sums over 32
 // terms at once) replace the eight v_mfma_f32_16x16x4_f32 (32 cycles each) of a
 // 16 x 16 x 32 product, and the sums round an eighth as often: against 64 bits
 // the outputs are closer than the fp32 matrix cores' (2-norm, 1024 x 1024 x 12 heads of 64,
 // N(0, 1): 2.3e-7 against 4.1e-7; 50 x 227 x 15: 2.0e-7 against 3.0e-7).
-// Scales: one per query row, one per tile for K, a running one per wave for V
-// (its accumulators are rescaled with it, as for a new maximum), 2^15 for the
-// weights; all powers of two, taken out again exactly.
+// Scales: one per query row, running ones per wave for K and V (V's accumulators
+// are rescaled with it, as for a new maximum), 2^15 for the weights; all powers
+// of two, taken out again exactly.
+//
+// What a shared scale does not carry goes to attn_block_f32, which computes the
+// block again from the inputs in plain fp32, 15 to 60 times slower (50 x 227 x 15
+// heads 9 -> 142 us): infinities in an operand and outputs that are not finite;
+// where a scale is set, a key's four columns of V 2^17 below the value that sets it
+// (as beside a masked row of padding that holds anything) and a largest query times
+// largest key that could add 2^14 to a score; at every tile, a column of V over a
+// lane's keys 2^18 below the scale. Of 400 calls with columns lognormal to 1.5, at most 6
+// take it. These checks, scores in the natural domain and masks after the scale cost
+// 4 to 7% (50 x 227 x 15 heads 8.5 -> 9.0 us, 690 x 690 x 12 block-causal 18.2 -> 19.2,
+// 1024 x 1024 x 12 22.8 -> 24.4).
 //
 // A block owns 16 * QF queries of one head and its W waves split the key
 // range in tiles of 32 keys (tile t, t + W, ...), each wave for all of the
@@ -546,10 +556,6 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 //                   float4 loads of eight key rows are its operands.
 // The loads of a wave's next tile are issued as soon as the registers of this
 // one are split.
-//
-// Infinities in an operand, outputs that are not finite and operands whose values
-// lie too far apart for one scale: such a block is computed again from the inputs
-// in plain fp32 (attn_block_f32).
 
 struct Split8 {
     f16x8 h, m;
@@ -1323,11 +1329,16 @@ void launch_split_w(const AttnArgs& a, hipStream_t st) {
 // (a block of 8 waves, or of 4 at head_dim 128, fills a CU's registers), else
 // the most: every fragment more divides the K/V traffic and the splitting, a
 // second round costs as much as the first. Measured, us (fp32 matrix cores |
-// QF 1, 2, 3, 4): 1024 x 1024 x 12 heads 43.7 | 34.3 31.5 36.1 25.6; 690 x 690
-// x 12, block-causal 28.8 | 26.2 22.3 20.1 28.0; 512 x 512 x 12 17.6 | 14.1
-// 12.8 13.5 15.3; 302 x 302 x 8 8.3 | 8.1 10.3 10.0 12.7.
-// W: 8 waves from 9 tiles of 32 keys on, 4 for 3 to 8 (50 x 227 x 15 heads 8.9
-// against 9.2), 2 below; head_dim 128 has the registers for 4.
+// QF 1, 2, 3, 4 at 8 waves): 1024 x 1024 x 12 heads 39.6 | 38.1 33.3 35.2 24.5; 690 x
+// 690 x 12, block-causal 26.1 | 27.7 23.5 19.1 25.6; 512 x 512 x 12 16.9 | 17.6
+// 12.3 13.0 15.3; 302 x 302 x 8 8.1 | 8.3 10.4 10.2 13.6; heads of 32: 1024 x 1024 x
+// 12 QF 1, 2, 4 37.6 33.2 25.2, 512 x 512 x 12 17.5 12.2 15.7; heads of 48: 1024 x 1024
+// x 8 26.6 18.2 24.4.
+// W: 8 waves from 9 tiles of 32 keys on, 4 for 3 to 8 (50 x 227 x 15 heads 9.0
+// against 9.2, heads of 32 x 8 7.0 against 7.4), 2 below (50 x 64 x 8 4.85 against
+// 4.98). head_dim 128 has the registers for 4: QF 1 or 2 at 4 waves | at 2, 302 x 302
+// x 8 13.3 17.0 | 17.2 21.8; 512 x 512 x 16 29.1 20.2 | 25.1 30.2; 1024 x 1024 x 8 45.3
+// 31.5 | 40.8 52.2; 50 x 64 x 8 7.2 9.8 | 7.0 9.4.
 template <int HDP, bool FULL>
 void run_split(const AttnArgs& a, hipStream_t st) {
     const int tiles = (a.seq_k + 31) / 32;
@@ -1350,7 +1361,8 @@ void run_split(const AttnArgs& a, hipStream_t st) {
     VLA_LAUNCH_CHECK();
 }
 
-// attn_fwd's waves: enough that each walks a few key tiles, at most 4 (LDS).
+// attn_fwd's waves, for heads of 129 to 256: enough that each walks a few key tiles,
+// at most 4 (LDS).
 void run_attn(const AttnArgs& a, hipStream_t st) {
     int kv = a.seq_k;
     if (a.mask_kind == 2) {  // keys no query of the problem can see are never walked
@@ -1385,10 +1397,9 @@ void launch_attention(const AttnArgs& a, hipStream_t st) {
                                      a.n_groups <= 256),
                 "attention: group mask needs q_group, k_group, allow and 1..256 groups");
     if (a.seq_q == 0) return;
-    // scale 0 (and non-finite scales) would turn a blocked score's -inf into
-    // NaN; lengths and strides past the block index's and offsets' range
-    const bool split = std::isfinite(a.scale) && a.scale != 0.0f && a.head_dim <= 128 && a.ldk < (1 << 24) &&
-                       a.ldv < (1 << 24) && (long)((a.seq_q + 15) / 16) * a.n_q < (1 << 20);
+    // (lengths and strides past the block index's and offsets' range)
+    const bool split = std::isfinite(a.scale) && a.head_dim <= 128 && a.ldk < (1 << 24) && a.ldv < (1 << 24) &&
+                       (long)((a.seq_q + 15) / 16) * a.n_q < (1 << 20);
     if (!split) run_attn(a, st);
     else if (a.head_dim == 64) run_split<64, true>(a, st);
     else if (a.head_dim < 64) run_split<64, false>(a, st);

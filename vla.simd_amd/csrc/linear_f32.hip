@@ -72,8 +72,12 @@ __device__ __forceinline__ float act_of(float v, int act) {
 // reach 2^6, or from the tile's where the row has none; the maxima of all
 // slabs are kept, and a tile some row of which ends up outside [2^3, 2^15] is
 // computed once more with the scales of the true maxima. So no part overflows
-// and no operand loses more than 2^-28 of its row's largest value (2^-22 of
-// itself at worst). Infinities are left to plain fmaf chains.
+// and an operand loses no more than 2^-22 of itself or 2^-28 of its row's largest
+// value. (Hence a row's last bits can depend on the other rows of its tile.)
+// Infinities are left to plain fmaf chains. Aimed at 2^12, a channel at 30 times the
+// others took the second pass: 690 x 768 x 3072 44.8 us against 27.1, 177 x 960 x 960
+// 16.9 against 10.0; at 2^6 rows 512 times their slab's maximum still do, at less
+// than twice the time.
 //
 // BM x BN tiles, four waves in a 2 x 2 grid. A K slab, KS steps of 32, is loaded as
 // float4 runs (whole 128-byte row segments per 8 lanes, 256 per 16 with KS = 2) into registers while
@@ -755,9 +759,11 @@ void launch_linear_f32(float* out, int ldo, const float* x, int ldx, const float
     if (few_tiles(M, N, K)) {
         // few tiles over a long K (ResNet's last stages): the split-K form,
         // 64-row x 16-column blocks whose 8 waves share K, so the chain of
-        // dependent loads per wave is an eighth of K (300 x 4608 x 512 48 us
-        // against 64, 302 x 3200 x 512 35 against 46; with 304 tiles of 32 x
-        // 32 the tiles are ahead: 1200 x 2304 x 256 36 against 49)
+        // dependent loads per wave is an eighth of K (300 x 4608 x 512, 160
+        // tiles of 32 x 32, 35.6 us against 43.3 in tiles; 177 x 2560 x 960, 180
+        // tiles, 21.7 against 26.3; 500 x 2048 x 448, 224, 18.2 against 22.1; near
+        // even at 302 x 2048 x 768, 240, 17.5 and 17.1; at 1200 x 2304 x 256, 304, the
+        // tiles are ahead, 26.7 against 35.0)
         const dim3 grid((N + 15) / 16, (M + 63) / 64);
         linear_f32_skinny<4, 8, true><<<grid, 512, 0, st>>>(out, ldo, x, ldx, W, ldw, bias, M, N, K, act,
                                                              accumulate, alpha);
