@@ -326,7 +326,11 @@ VLA_API int64_t vla_h2d_bytes(int32_t weights_only);
  * head, kv head = h / (n_q / n_kv); a key with mask == lowest() or score -inf
  * has weight 0; a row with every key blocked is the uniform mean of V.
  * mask [seq_q, seq_k] additive, NULL = dense (gqa_attention_dense,
- * lm_ops.h:43, common/attn.cpp:23-28). head_dim <= 256, head_dim % 4 == 0. */
+ * lm_ops.h:43, common/attn.cpp:23-28). head_dim <= 256, head_dim % 4 == 0.
+ * Up to head_dim 128 the products take 22 bits of every operand, with smaller
+ * errors than fp32 sums of ordinary inputs have. Queries whose keys or values lie
+ * too far apart in size for that (infinities, masked rows of padding 2^17 above the
+ * others) are computed in plain fp32, 15 to 60 times slower. */
 VLA_API int32_t vla_gqa_attention_masked(float* out, const float* Q, const float* K,
                                          const float* V, int32_t seq_q, int32_t seq_k,
                                          int32_t n_q, int32_t n_kv, int32_t head_dim,

@@ -3,8 +3,9 @@
 Query fragments per block (1 to 4) and waves (2, 4, 8) follow from the sizes;
 the sizes here lie on both sides of each of those lines, of the 16-query and
 32-key tiles and of the head widths. Against double-precision softmax: the
-parts keep every operand to 2^-22 of itself at worst, so the outputs are held
-to what fp32 sums give (2e-6 of the result's 2-norm; about 2e-7 is seen).
+parts keep every operand to 2^-22 of itself or 2^-40 of the largest that shares
+its scale, so the outputs are held to what fp32 sums give (2e-6 of the result's
+2-norm; about 2e-7 is seen).
 """
 
 import math

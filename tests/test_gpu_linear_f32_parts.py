@@ -2,7 +2,7 @@
 wrong: both sides of every tile choice, ragged rows, columns and K slabs,
 unaligned rows, and rows whose scale the guess from one slab does not give.
 Against float64, per output row: a row's parts keep 2^-22 of every value or
-2^-33 of the row's largest, so a row's error stays what fp32 sums give
+2^-28 of the row's largest, so a row's error stays what fp32 sums give
 (a few 2^-24 sqrt(K) of |x||w|; 2e-6 of the row's 2-norm bound is held).
 """
 

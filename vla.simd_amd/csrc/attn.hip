@@ -516,7 +516,8 @@ void launch_w(const AttnArgs& a, hipStream_t st) {
 // attn_split: the same attention with both products on the fp16 matrix cores.
 //
 // The operands' two parts (fp16parts.h) hold them to 2^-22 (2^-24.5 in the mean)
-// or to 2^-40 of the largest value that shares the scale, whichever is more. So three
+// or to 2^-40 of the largest value that shares the scale, whichever is more (a
+// weight under 2^-41 of its query's largest adds nothing to the values' sum). So three
 // v_mfma_f32_16x16x32_f16 (16 cycles each, exact products, fp32 sums over 32
 // terms at once) replace the eight v_mfma_f32_16x16x4_f32 (32 cycles each) of a
 // 16 x 16 x 32 product, and the sums round an eighth as often: against 64 bits
