@@ -267,3 +267,23 @@ def test_operands_of_mixed_sizes(vla):
     want = naive(Q / dims, K * dims, V * cols, sq, sk, 2, 2, HD, 0.125)
     err = np.linalg.norm(got - want, axis=0) / np.linalg.norm(want, axis=0)
     assert err.max() < 4e-6, err.max()
+
+
+@pytest.mark.parametrize("sq,sk,nq,hd", [(40, 60, 2, 64), (40, 100, 2, 64), (1400, 70, 12, 64), (40, 300, 2, 64), (400, 290, 12, 64),
+                                         (700, 290, 12, 64), (1040, 290, 12, 64), (1100, 300, 12, 32), (40, 90, 3, 128),
+                                         (600, 90, 8, 100)])
+@pytest.mark.parametrize("kind", ["none", "causal", "groups", "dense"])
+def test_plain_form_of_every_block_shape(vla, sq, sk, nq, hd, kind):
+    """One infinite value of V sends every block of its head to the plain form, at each
+    count of queries and waves per block; the other columns are what they are without."""
+    Q, K, V = qkv(sq + hd, sq, sk, nq, nq, hd)
+    kw, keep = masks_of(vla, kind, sq, sk)
+    scale = 1 / math.sqrt(hd)
+    want = naive(Q, K, V, sq, sk, nq, nq, hd, scale, np.where(keep, 0, -np.inf).astype(np.float32))
+    V[0, hd + 3] = np.inf  # head 1
+    got = vla.attention(Q, K, V, nq, nq, hd, scale, **kw)
+    rest = np.arange(nq * hd) != hd + 3
+    assert rel(got[:, rest], want[:, rest]) < 2e-6
+    sees = keep[:, 0] | ~keep.any(axis=1)
+    assert not np.isfinite(got[sees, hd + 3]).any()
+    assert np.isfinite(got[~sees, hd + 3]).all()
